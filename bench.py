@@ -79,8 +79,8 @@ PERSISTENT_KERNEL = "j3d_star1_persistent_kernel"
 # Files that define the persistent 7-point kernel and its launch: a recorded
 # profile applies only while their contents are unchanged.
 KERNEL_SOURCES = ["perks_amd/csrc/j3d_persistent_kernel.h", "perks_amd/csrc/j3d_persistent.hip",
-                  "perks_amd/csrc/j3d_persistent_f64.hip", "perks_amd/csrc/j3d_persistent.h",
-                  "perks_amd/csrc/grid_sync.h", "perks_amd/csrc/perks_device.h", "perks_amd/csrc/j3d_common.h",
+                  "perks_amd/csrc/j3d_persistent_f64.hip", "perks_amd/csrc/j3d_persistent_f64_shared.hip",
+                  "perks_amd/csrc/j3d_persistent.h", "perks_amd/csrc/grid_sync.h", "perks_amd/csrc/perks_device.h", "perks_amd/csrc/j3d_common.h",
                   "perks_amd/csrc/storage16.h", "perks_amd/csrc/storage_fmt.h", "perks_amd/build.py"]
 SIMDS, SHADER_ENGINES = 1024, 32  # MI355X: 256 CUs x 4 SIMDs; 8 XCDs x 4 SEs
 

@@ -777,10 +777,10 @@ __global__ void __launch_bounds__(kLanes) cg_persistent_kernel(CgArgs<V> a)
     // ---- r = b + (-1) * A x ; partials of r.r and b.b ----
     phase_initial<V, FMT>(a, c, me, kb, true, lds);
     bool fill = a.x_is_zero != 0;  // the first SpMV fills the matrix cache
-    if (!grid_sync(a.sync, G, a.timeout)) return;
+    if (!grid_sync(a.sync, G, a.timeout, true)) return;
     if (has_long && !a.x_is_zero) {
         fix_initial<V, FMT>(a, c, me, lds);
-        if (!grid_sync(a.sync, G, a.timeout)) return;
+        if (!grid_sync(a.sync, G, a.timeout, false)) return;
     }
     double r1 = reduce_parts(a.part_a, a.nseg, lds);
     const double bbv = reduce_parts(a.part_b, a.nseg, lds);
@@ -789,7 +789,7 @@ __global__ void __launch_bounds__(kLanes) cg_persistent_kernel(CgArgs<V> a)
         if (a.hist && a.hist_cap > 0) a.hist[0] = r1;
         *a.bb_out = bbv;
     }
-    if (!grid_sync(a.sync, G, a.timeout)) return;  // part_a/part_b are rewritten below
+    if (!grid_sync(a.sync, G, a.timeout, false)) return;  // part_a/part_b are rewritten below
 
     double r0 = 0.0;
     int k = 1;
@@ -800,16 +800,16 @@ __global__ void __launch_bounds__(kLanes) cg_persistent_kernel(CgArgs<V> a)
         if (k == 1) phase_spmv<V, FMT, true>(a, c, me, kb, pold, pnew, (V)0, fill, lds);
         else phase_spmv<V, FMT, false>(a, c, me, kb, pold, pnew, (V)(r1 / r0), fill, lds);
         fill = false;
-        if (!grid_sync(a.sync, G, a.timeout)) return;
+        if (!grid_sync(a.sync, G, a.timeout, false)) return;
         if (has_long) {
             fix_spmv<V, FMT>(a, c, me, pnew, lds);
-            if (!grid_sync(a.sync, G, a.timeout)) return;
+            if (!grid_sync(a.sync, G, a.timeout, false)) return;
         }
         const double pap = reduce_parts(a.part_a, a.nseg, lds);
         const double alpha_d = r1 / pap;
         // ---- x = alpha*p + x ; r = (-alpha)*Ap + r ; partials of r.r ----
         phase_update<V, FMT>(a, c, me, pnew, (V)alpha_d, lds);
-        if (!grid_sync(a.sync, G, a.timeout)) return;
+        if (!grid_sync(a.sync, G, a.timeout, false)) return;
         r0 = r1;
         r1 = reduce_parts(a.part_b, a.nseg, lds);
         if (me == 0 && t == 0 && a.hist && k < a.hist_cap) a.hist[k] = r1;

@@ -192,7 +192,7 @@ __global__ void __launch_bounds__(256) j2d_kernel(J2dArgs a, KCoefs cf)
                 }
             }
         }
-        if (pass + 1 < a.npass && !grid_sync(a.sync, G, a.timeout)) return;
+        if (pass + 1 < a.npass && !grid_sync(a.sync, G, a.timeout, pass == 0)) return;
     }
 }
 

@@ -619,7 +619,7 @@ __global__ void __launch_bounds__(kWaves * 64) j2d_stream_kernel(J2dArgs a, KCoe
                 }
             }
         }
-        if (pass + 1 < a.npass && !grid_sync(a.sync, G, a.timeout)) return;
+        if (pass + 1 < a.npass && !grid_sync(a.sync, G, a.timeout, pass == 0)) return;
     }
 }
 

@@ -207,7 +207,7 @@ __global__ void __launch_bounds__(kThreads) j3g_kernel(J3gArgs a, KCoefs cf)
                 }
             }
         }
-        if (pass + 1 < a.npass && !grid_sync(a.sync, G, a.timeout)) return;
+        if (pass + 1 < a.npass && !grid_sync(a.sync, G, a.timeout, pass == 0)) return;
     }
 }
 

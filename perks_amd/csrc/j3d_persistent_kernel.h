@@ -901,7 +901,7 @@ j3d_star1_persistent2_kernel(typename Elem<FMT>::S* buf_a, typename Elem<FMT>::S
         S* t = src;
         src = dst;
         dst = t;
-        if (pass + 1 < npass && !grid_sync(a.sync, gridDim.x, a.timeout)) return;
+        if (pass + 1 < npass && !grid_sync(a.sync, gridDim.x, a.timeout, pass == 0)) return;
     }
 }
 
@@ -965,7 +965,7 @@ j3d_star1_persistent_kernel(typename Elem<FMT>::S* buf_a, typename Elem<FMT>::S*
         S* t = src;
         src = dst;
         dst = t;
-        if (pass + 1 < npass && !grid_sync(a.sync, gridDim.x, a.timeout)) return;
+        if (pass + 1 < npass && !grid_sync(a.sync, gridDim.x, a.timeout, pass == 0)) return;
     }
 }
 
@@ -1033,6 +1033,18 @@ void* pick_bc(int bc, bool has_div, int var)
     return has_div ? pick_variant<FMT, PERKS_BC_CLAMP, true, SR, UP>(var)
                    : pick_variant<FMT, PERKS_BC_CLAMP, false, SR, UP>(var);
 }
+
+// These instantiations are compiled in files of their own
+// (j3d_persistent_<fmt>[_sr][_shared].hip), so that a build runs them in
+// parallel; the rest of a format's in j3d_persistent_<fmt>.hip.
+extern template void* pick_bc<PERKS_F64, false, kUpdShared>(int, bool, int);
+extern template void* pick_bc<PERKS_F32, false, kUpdShared>(int, bool, int);
+extern template void* pick_bc<PERKS_F16, false, kUpdShared>(int, bool, int);
+extern template void* pick_bc<PERKS_F16, true, kUpdGold>(int, bool, int);
+extern template void* pick_bc<PERKS_F16, true, kUpdShared>(int, bool, int);
+extern template void* pick_bc<PERKS_BF16, false, kUpdShared>(int, bool, int);
+extern template void* pick_bc<PERKS_BF16, true, kUpdGold>(int, bool, int);
+extern template void* pick_bc<PERKS_BF16, true, kUpdShared>(int, bool, int);
 
 // sr: stochastic rounding (16-bit storage only; FP64/FP32 ignore it).
 // up: the update form (kUpd*); the fused form is built for FP64/FP32 storage

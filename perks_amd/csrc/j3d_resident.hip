@@ -270,7 +270,7 @@ j3d_star1_resident_kernel(T* buf_a, T* buf_b, ResArgs a, KCoefs cf)
             m.step(src);
             m.store(dst, last);
         }
-        if (!last && !grid_sync(a.sync, gridDim.x, a.timeout)) return;
+        if (!last && !grid_sync(a.sync, gridDim.x, a.timeout, t == 0)) return;
     }
 }
 

@@ -341,7 +341,7 @@ __global__ void __launch_bounds__(kWaves * 64) j3s_kernel(J3gArgs a, KCoefs cf)
             if (L <= 1 || LM < 2) go(std::integral_constant<int, 1>{});
             else if constexpr (LM >= 2) go(std::integral_constant<int, 2>{});
         }
-        if (pass + 1 < a.npass && !grid_sync(a.sync, G, a.timeout)) return;
+        if (pass + 1 < a.npass && !grid_sync(a.sync, G, a.timeout, pass == 0)) return;
     }
 }
 
