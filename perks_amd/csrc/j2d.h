@@ -26,7 +26,7 @@ struct J2dGrid {
     int steps;
     int tiles;
     int item_end;
-    int seg;  // rows per segment (streaming kernel, tile variant 2)
+    int seg0, seg;  // streaming kernel: rows of the first segment, and of each following one
 };
 
 struct J2dArgs {
@@ -59,6 +59,13 @@ void* j2d_kernel_bf16(int shape, int bc, bool has_div, int tile);
 __host__ __device__ constexpr int stream_max_levels(int radius)
 {
     return radius == 1 ? 4 : (radius == 2 ? 2 : 1);
+}
+
+// Rows per loop trip of the row-streaming kernel, and rows it loads ahead: at
+// least 8, a multiple of the 2R+1 rows of a level's window.
+__host__ __device__ constexpr int stream_trip(int radius)
+{
+    return (2 * radius + 1) * ((8 + 2 * radius) / (2 * radius + 1));
 }
 
 // Ghost columns per side of a two-column streaming strip: R*L rounded up to even.

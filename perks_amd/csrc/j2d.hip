@@ -49,7 +49,6 @@ constexpr int kStreamTile = 2;     // tile variant of the row-streaming kernel, 
 constexpr int kPairTile = 4;       // the row-streaming kernel, two columns per lane
 constexpr int kDefaultTile = -1;   // resolved per run: kPairTile where it applies, else kStreamTile
 constexpr int kStreamWaves = 4;    // its waves per workgroup, one work item each
-constexpr int kStreamItems = 16384;  // work items a launch aims for (segments are cut to reach it)
 
 void* kernel_for(int dtype, int shape, int bc, bool hd, int tile)
 {
@@ -160,21 +159,119 @@ struct Work {
     long long cell_steps = 0;
 };
 
-int build_work(const J2dSpec* specs, int n, int R, int tx, int ty, int L, Work* w)
+// The kernel of a configuration and how many workgroups of it are resident at
+// once: the persistent grid's size, or what a per-step launch fills.
+struct Resident {
+    void* fn = nullptr;
+    int cus = 0;
+    int occ = 0;  // workgroups per CU
+    long long waves() const { return (long long)cus * occ * kStreamWaves; }
+};
+
+int resident(int dtype, const perks_stencil_opts* o, const KCoefs& cf, const Config& c, Resident* out)
 {
+    perks_device_caps caps;
+    int rc = device_caps_cached(&caps);
+    if (rc != PERKS_OK) return rc;
+    out->cus = caps.cu_count;
+    out->fn = kernel_for(dtype, o->shape, o->boundary, cf.divisor != 0.0, c.tile);
+    if (!out->fn) return PERKS_ERR_UNSUPPORTED;
+    int occ = 0;
+    PERKS_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void*>(out->fn), 256, 0));
+    if (occ <= 0) return PERKS_ERR_NOT_LAUNCHABLE;
+    if (o->method != PERKS_METHOD_PLAIN) {
+        occ = std::min(occ, kCoopMaxWavesPerCu / 4);  // 256-thread workgroups
+        if (o->blkpsm > 0 && o->blkpsm < occ) occ = o->blkpsm;
+        if (c.occ > 0 && c.occ < occ) occ = c.occ;
+    }
+    out->occ = occ;
+    return PERKS_OK;
+}
+
+// Cuts a strip of ny rows into segments for the streaming kernel: the first of
+// seg0 rows, the following of `seg`, the last of what is left.  Segments at the
+// top and bottom faces run the form of the kernel with the boundary rules, so
+// they get the smaller ones: half of what whole segments leave over, and at
+// least enough (edge rows, more than the ghost rows) that the others' ghost
+// rows lie inside the grid.
+struct RowCut {
+    int seg0, seg;
+    long long count(int ny) const { return 1 + ((long long)ny - seg0 + seg - 1) / seg; }
+};
+RowCut cut_rows(int ny, int seg, int edge)
+{
+    if (ny <= seg) return {ny, seg};
+    const int rest = ny > 2 * edge ? (ny - 2 * edge) % seg + 2 * edge : ny;  // rows of the first and last segments
+    return {(rest + 1) / 2, seg};
+}
+
+// Rows per segment of the streaming kernel: the height that makes a pass
+// shortest, among those whose rows (seg + 2RL with the ghost rows) fill whole
+// trips of stream_trip(R) rows.
+//   Persistent: the resident waves take as many rounds as the items need, each
+//   of a segment's rows and the time until its first loads have arrived (about
+//   2 us, which is 150 / (L * points) rows' arithmetic).  8192^2 FP32 2d9pt, 4
+//   steps per pass: one round of 154 rows, 29.4 ms for 500 steps; four rounds of
+//   37 rows take 31.1.
+//   Per step: a CU's workgroups run together and share its bandwidth, so what
+//   counts is the rows of the CU that gets most, two rows' time for starting
+//   each item, and that one workgroup alone hides no latency.  2048^2 FP64
+//   2d5pt: 25 rows (3 workgroups per CU) 13.0 us per step, 43 rows (2) 13.5,
+//   16 rows (5) 16.8, 7 rows (10) 16.0.
+int stream_segment(const J2dSpec* specs, int n, int R, int npts, int L, int VW, int edge, bool plain,
+                   const Resident& res)
+{
+    const int trip = stream_trip(R), ghost = 2 * R * L;
+    const int fill = 150 / (L * npts);
+    int most = 1;
+    for (int i = 0; i < n; ++i)
+        if (specs[i].steps > 0) most = std::max(most, specs[i].ny);
+    int best = 1;
+    double best_cost = 1e300;
+    // (a coarser walk over the heights of a batch: its grids average them out)
+    for (long long k = ghost / trip + 1;; k += 1 + k / (n == 1 ? 16 : 4)) {
+        const int seg = (int)std::min<long long>(k * trip - ghost, 0x7fffffffLL);
+        long long items = 0, passes = 1;  // over all passes
+        for (int i = 0; i < n; ++i) {
+            if (specs[i].steps <= 0) continue;
+            const long long np = n == 1 ? 1 : (specs[i].steps + L - 1) / L;
+            items += (specs[i].nx + VW - 1LL) / VW * cut_rows(specs[i].ny, seg, edge).count(specs[i].ny) * np;
+            passes = std::max(passes, np);
+        }
+        double cost;
+        if (plain) {
+            const long long per_pass = 4LL * res.cus * passes;
+            const double wgs = (double)((items + per_pass - 1) / per_pass);
+            cost = (wgs + 0.5) * ((double)seg + ghost + 2);
+        } else {
+            // half a round is lost at the end of each pass of several grids
+            const double rounds = (double)((items + res.waves() - 1) / res.waves()) + (n == 1 ? 0.0 : 0.5 * passes);
+            cost = rounds * ((double)seg + ghost + fill);
+        }
+        if (cost < best_cost * (1 - 1e-9)) {
+            best_cost = cost;
+            best = seg;
+        }
+        if (seg >= most) break;
+    }
+    return best;
+}
+
+int build_work(const J2dSpec* specs, int n, const ShapeDesc& sd, int tx, int ty, int L, bool plain,
+               const Resident& res, Work* w)
+{
+    const int R = sd.radius;
     const bool stream = ty == 0;
     const int VW = (stream && tx == 128) ? 128 - 2 * pair_ghost(R, L) : tx - 2 * R * L;
     int VH = ty - 2 * R * L;
     if (VW < 1 || (!stream && VH < 1)) return PERKS_ERR_INVALID_ARG;
+    const int edge = 2 * R * L + 1;  // fewest rows of a strip's first and last segment
     if (stream) {
-        // Segment height: enough work items to fill the chip, and at least
-        // 8*R*L rows so that the ghost rows stay a small part of an item.
-        long long strip_rows = 0;
+        int npts = 0;
+        for (int g = 0; g < sd.ngroups; ++g) npts += sd.g[g].npts;
         for (int i = 0; i < n; ++i)
-            if (specs[i].steps > 0 && specs[i].nx > 0 && specs[i].ny > 0)
-                strip_rows += (long long)((specs[i].nx + VW - 1) / VW) * specs[i].ny;
-        const long long seg = std::max<long long>(8LL * R * L, (strip_rows + kStreamItems - 1) / kStreamItems);
-        VH = (int)std::min<long long>(seg, 0x7fffffffLL);
+            if (specs[i].ny <= 0 || specs[i].nx <= 0) return PERKS_ERR_INVALID_ARG;
+        VH = stream_segment(specs, n, R, npts, L, VW, edge, plain, res);
     }
     std::vector<int> order(n);
     for (int i = 0; i < n; ++i) order[i] = i;
@@ -191,7 +288,9 @@ int build_work(const J2dSpec* specs, int n, int R, int tx, int ty, int L, Work* 
         if (s.steps == 0) continue;
         // Tiles are laid out with the full-pass geometry; a shorter last pass
         // reuses them (a smaller ghost rim is enough for it).
-        const long long tiles = (long long)((s.nx + VW - 1) / VW) * ((s.ny + VH - 1) / VH);
+        const RowCut cut = stream ? cut_rows(s.ny, VH, edge) : RowCut{0, 0};
+        const long long tiles =
+            (long long)((s.nx + VW - 1) / VW) * (stream ? cut.count(s.ny) : (long long)((s.ny + VH - 1) / VH));
         if (w->items + tiles > 0x7fffffffLL) return PERKS_ERR_UNSUPPORTED_SIZE;
         J2dGrid g;
         g.a = s.a;
@@ -200,7 +299,8 @@ int build_work(const J2dSpec* specs, int n, int R, int tx, int ty, int L, Work* 
         g.nx = s.nx;
         g.steps = s.steps;
         g.tiles = (int)tiles;
-        g.seg = stream ? VH : 0;
+        g.seg0 = cut.seg0;
+        g.seg = cut.seg;
         w->items += g.tiles;
         g.item_end = w->items;
         w->grids.push_back(g);
@@ -264,14 +364,10 @@ struct Launch {
     KCoefs cf;
 };
 
-int prepare_launch(int dtype, const perks_stencil_opts* o, const KCoefs& cf, const Config& c, const Work& w,
-                   const DeviceWork& dw, GridSync* gs, Launch* out)
+void prepare_launch(int dtype, const perks_stencil_opts* o, const KCoefs& cf, const Config& c, const Resident& r,
+                    const Work& w, const DeviceWork& dw, GridSync* gs, Launch* out)
 {
-    perks_device_caps caps;
-    int rc = device_caps_cached(&caps);
-    if (rc != PERKS_OK) return rc;
-    out->fn = kernel_for(dtype, o->shape, o->boundary, cf.divisor != 0.0, c.tile);
-    if (!out->fn) return PERKS_ERR_UNSUPPORTED;
+    out->fn = r.fn;
     out->tile = c.tile;
     std::memset(&out->args, 0, sizeof(out->args));
     out->args.grids = dw.grids;
@@ -285,18 +381,11 @@ int prepare_launch(int dtype, const perks_stencil_opts* o, const KCoefs& cf, con
     out->occ = 0;
     out->grid = 0;
     if (o->method != PERKS_METHOD_PLAIN) {
-        int occ = 0;
-        PERKS_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void*>(out->fn), 256, 0));
-        if (occ <= 0) return PERKS_ERR_NOT_LAUNCHABLE;
-        occ = std::min(occ, kCoopMaxWavesPerCu / 4);  // 256-thread workgroups
-        if (o->blkpsm > 0 && o->blkpsm < occ) occ = o->blkpsm;
-        if (c.occ > 0 && c.occ < occ) occ = c.occ;
-        out->occ = occ;
-        out->grid = std::min(caps.cu_count * occ, groups_for(c.tile, w.items));
+        out->occ = r.occ;
+        out->grid = std::min(r.cus * r.occ, groups_for(c.tile, w.items));
         out->args.npass = w.npass;
         out->args.step_offset = 0;
     }
-    return PERKS_OK;
 }
 
 // Enqueues the launch(es) on `stream`.  cooperative: hipLaunchCooperativeKernel
@@ -387,7 +476,10 @@ int j2d_run(int dtype, J2dSpec* specs, int n, const perks_stencil_opts* o, hipSt
     int tx, ty;
     tile_dims(dtype, c.tile, &tx, &ty);
     Work w;
-    rc = build_work(specs, n, sd->radius, tx, ty, c.levels, &w);
+    Resident res;
+    rc = resident(dtype, o, cf, c, &res);
+    if (rc != PERKS_OK) return rc;
+    rc = build_work(specs, n, *sd, tx, ty, c.levels, o->method == PERKS_METHOD_PLAIN, res, &w);
     if (rc != PERKS_OK) return rc;
     for (int i = 0; i < n; ++i) specs[i].result_in_b = w.result_in_b[i];
     if (w.grids.empty()) {
@@ -405,8 +497,7 @@ int j2d_run(int dtype, J2dSpec* specs, int n, const perks_stencil_opts* o, hipSt
     if (rc != PERKS_OK) return rc;
     GridSync* gs = lease.gs;
     Launch l;
-    rc = prepare_launch(dtype, o, cf, c, w, g_work[dev], gs, &l);
-    if (rc != PERKS_OK) return rc;
+    prepare_launch(dtype, o, cf, c, res, w, g_work[dev], gs, &l);
 
     hipEvent_t ev0, ev1;
     PERKS_HIP_TRY(hipEventCreate(&ev0));
@@ -490,7 +581,10 @@ int j2d_run_noalloc(int dtype, J2dSpec* specs, int n, const perks_stencil_opts* 
     int tx, ty;
     tile_dims(dtype, c.tile, &tx, &ty);
     Work w;
-    rc = build_work(specs, n, sd->radius, tx, ty, c.levels, &w);
+    Resident res;
+    rc = resident(dtype, o, cf, c, &res);
+    if (rc != PERKS_OK) return rc;
+    rc = build_work(specs, n, *sd, tx, ty, c.levels, o->method == PERKS_METHOD_PLAIN, res, &w);
     if (rc != PERKS_OK) return rc;
     if (w.grids.size() > (size_t)PERKS_NOALLOC_MAX_GRIDS || w.active.size() > (size_t)PERKS_NOALLOC_MAX_PASSES) {
         std::fprintf(stderr,
@@ -521,8 +615,7 @@ int j2d_run_noalloc(int dtype, J2dSpec* specs, int n, const perks_stencil_opts* 
     PERKS_HIP_TRY(hipMemcpyAsync(dw.active, w.active.data(), sizeof(int) * w.active.size(), hipMemcpyHostToDevice,
                                  stream));
     Launch l;
-    rc = prepare_launch(dtype, o, cf, c, w, dw, gs, &l);
-    if (rc != PERKS_OK) return rc;
+    prepare_launch(dtype, o, cf, c, res, w, dw, gs, &l);
     rc = enqueue(l, o, w, stream, true);
     if (rc != PERKS_OK) return rc;
     // Wait before the scratch can be rewritten by the next call.
@@ -594,22 +687,25 @@ int mark_cooperative(hipGraph_t g)
 // Times one configuration on scratch buffers: every grid runs min(steps, cap)
 // steps.  Returns cells per second (0 when the configuration does not apply).
 double time_config(int dtype, const perks_stencil_opts* o, const KCoefs& cf, const Config& c,
-                   const std::vector<J2dSpec>& scratch, int R, int cap, hipStream_t stream, GridSync* gs)
+                   const std::vector<J2dSpec>& scratch, const ShapeDesc& sd, int cap, hipStream_t stream, GridSync* gs)
 {
     int tx, ty;
     tile_dims(dtype, c.tile, &tx, &ty);
-    if (c.levels > max_levels(dtype, c.tile, R)) return 0.0;
+    if (c.levels > max_levels(dtype, c.tile, sd.radius)) return 0.0;
     std::vector<J2dSpec> specs = scratch;
     for (auto& s : specs) s.steps = std::min(s.steps, cap);
     Work w;
-    if (build_work(specs.data(), (int)specs.size(), R, tx, ty, c.levels, &w) != PERKS_OK || w.grids.empty())
+    Resident res;
+    if (resident(dtype, o, cf, c, &res) != PERKS_OK) return 0.0;
+    if (build_work(specs.data(), (int)specs.size(), sd, tx, ty, c.levels, o->method == PERKS_METHOD_PLAIN, res,
+                   &w) != PERKS_OK || w.grids.empty())
         return 0.0;
     DeviceWork dw;
     double best = 0.0;
     do {
         if (dw.upload(w, stream) != PERKS_OK) break;
         Launch l;
-        if (prepare_launch(dtype, o, cf, c, w, dw, gs, &l) != PERKS_OK) break;
+        prepare_launch(dtype, o, cf, c, res, w, dw, gs, &l);
         hipEvent_t e0, e1;
         if (hipEventCreate(&e0) != hipSuccess) break;
         if (hipEventCreate(&e1) != hipSuccess) {
@@ -701,7 +797,7 @@ int plan_batch(int dtype, const perks_grid2d* grids, int ngrids, const perks_ste
             for (int L : level_choices)
                 for (int occ : occ_choices) {
                     const Config c{tl, L, occ};
-                    const double v = time_config(dtype, o, cf, c, scratch, sd->radius, kTuneSteps, stream, p->gs);
+                    const double v = time_config(dtype, o, cf, c, scratch, *sd, kTuneSteps, stream, p->gs);
                     if (v > best) {
                         best = v;
                         best_c = c;
@@ -717,9 +813,13 @@ int plan_batch(int dtype, const perks_grid2d* grids, int ngrids, const perks_ste
 
     int tx, ty;
     tile_dims(dtype, p->cfg.tile, &tx, &ty);
-    rc = build_work(specs.data(), ngrids, sd->radius, tx, ty, p->cfg.levels, &p->work);
+    Resident res;
+    rc = resident(dtype, o, cf, p->cfg, &res);
+    if (rc == PERKS_OK)
+        rc = build_work(specs.data(), ngrids, *sd, tx, ty, p->cfg.levels, o->method == PERKS_METHOD_PLAIN, res,
+                        &p->work);
     if (rc == PERKS_OK) rc = p->dw.upload(p->work, stream);
-    if (rc == PERKS_OK) rc = prepare_launch(dtype, o, cf, p->cfg, p->work, p->dw, p->gs, &p->launch);
+    if (rc == PERKS_OK) prepare_launch(dtype, o, cf, p->cfg, res, p->work, p->dw, p->gs, &p->launch);
     if (rc == PERKS_OK && hipStreamSynchronize(stream) != hipSuccess) rc = PERKS_ERR_HIP;
     if (rc == PERKS_OK && !p->work.grids.empty()) {
         // Capture the launch(es) on a stream of our own (default priority).

@@ -2,9 +2,9 @@
 // registers (tile variant 2; instantiated per storage type in
 // j2d_stream_{f64,f32,f16,bf16}.hip).
 //
-// A work item is a strip of 64 columns (one per lane) and a segment of rows
-// of one grid; each wave runs its own items, so there is no LDS and no
-// workgroup barrier.  The wave marches down the segment one row per
+// A work item is a strip of 64 columns (one per lane; two per lane: 128) and
+// a segment of rows of one grid; each wave runs its own items, so there is no
+// LDS and no workgroup barrier.  The wave marches down the segment one row per
 // iteration: level 0 is the field row read from HBM (requested D rows ahead
 // and kept as loaded until it enters the window, where it is widened, so
 // nothing waits on a load before its first use), and level l (1..L) computes
@@ -18,13 +18,14 @@
 //
 // Boundaries: at every level, the cells just outside the grid hold what the
 // boundary rule reads there -- 0 (zero) or the nearest edge cell (clamp) --
-// so the update itself never tests for a face.  Level 0 gets them from
-// clamped loads (zeroed as the row enters the window); higher levels copy the edge row into the rows
-// beyond the top and bottom faces when the edge row is produced, and the
-// edge column into the lanes beyond the side faces (readlane).  This is the
-// per-step kernel's rule applied level by level, so a pass equals L stored
-// steps bit for bit: arithmetic is the shape table in order without FMA
-// contraction (eval_shape) and every level is rounded to the storage format.
+// so the update itself never tests for a face.  Level 0 gets them from its
+// loads; higher levels copy the edge row into the rows beyond the top and
+// bottom faces when the edge row is produced, and the edge column into the
+// lanes beyond the side faces (readlane).  Items that touch no face run a form
+// without any of it.  This is the per-step kernel's rule applied level by
+// level, so a pass equals L stored steps bit for bit: arithmetic is the shape
+// table in order without FMA contraction (eval_shape) and every level is
+// rounded to the storage format.
 #pragma once
 
 #include <type_traits>
@@ -40,6 +41,12 @@ using j2dk::eval_shape;
 using j2dk::shape_desc;
 
 constexpr int kWaves = 4;  // waves per workgroup (each runs its own items)
+
+// Wave-uniform conditions that few rows meet: what they guard opens with
+// keep_branch(), which the compiler may not execute speculatively, so it stays
+// behind a branch instead of becoming a select per held value, level and row.
+__device__ __forceinline__ bool rarely(bool c) { return __builtin_expect_with_probability(c, 0, 0.9999); }
+__device__ __forceinline__ void keep_branch() { asm volatile(""); }
 
 // sh[R + dx] = the row value at column x + dx, for dx in [-R, R]: lane i
 // receives lane i-1 (west) or lane i+1 (east), repeatedly.
@@ -65,252 +72,6 @@ __device__ __forceinline__ double read_lane(double v, int l)
     const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(u >> 32), l);
     return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
-
-template <int SHAPE, typename S, int BC, bool HAS_DIV, int L>
-struct Strip {
-    using C = typename Fmt<S>::C;
-    static constexpr const ShapeDesc& SD = shape_desc<SHAPE>();
-    static constexpr int R = SD.radius;
-    static constexpr bool BOX = SD.is_box != 0;
-    static constexpr int Q = 2 * R + 1;            // rows of a level's window
-    static constexpr int D = Q * ((8 + Q - 1) / Q);  // level-0 rows loaded ahead (at least 8, a multiple of Q)
-    static constexpr int UF = D;  // stages per loop trip: a multiple of Q and D, so every ring slot is static
-    static constexpr int NS = BOX ? Q : 1;
-
-    const S* src;
-    S* dst;
-    int nx, ny;
-    int x, xc;       // this lane's column, clamped into the grid
-    bool xout;       // the column lies outside the grid
-    bool xedge;      // the strip reaches past a side face
-    int lane_w, lane_e;  // lanes of columns 0 and nx-1 (clamped into the wave)
-    bool st_ok;      // this lane stores its column
-    int lo[L + 1], hi[L + 1];
-    int ys, ye;
-    C k[kMaxGroups];
-    double kd[kMaxGroups];
-    double kdiv;
-    bool sr;
-    uint32_t key[L + 1];
-
-    using Raw = typename Fmt<S>::Raw;
-    Raw fl[D];        // level-0 rows in flight, as loaded (row i in slot (i - i0) mod D)
-    C win[L][Q][NS];  // level l's window; boxes keep the x shifts
-
-    static constexpr int mq(int a) { return ((a % Q) + Q) % Q; }
-
-    __device__ __forceinline__ Raw load(int q) const
-    {
-        const int qc = q < 0 ? 0 : (q >= ny ? ny - 1 : q);
-        return Fmt<S>::ld_raw(src + (size_t)qc * nx, (size_t)xc);
-    }
-
-    // Row q of level 0 from its loaded word, at its first use (D rows after
-    // its load was issued): widened, and 0 outside the grid (zero boundary).
-    __device__ __forceinline__ C arrive(int q, Raw w) const
-    {
-        const C v = Fmt<S>::widen(w);
-        if constexpr (BC == PERKS_BC_ZERO) return (q < 0 || q >= ny || xout) ? (C)0 : v;
-        return v;
-    }
-
-    // Level LV's row at relative slot index `rel` (static), column offset dx.
-    template <int LV>
-    __device__ __forceinline__ C cell(int rel, int dx, const C (&csh)[Q], int centre_rel) const
-    {
-        if constexpr (BOX) return win[LV][mq(rel)][R + dx];
-        else {
-            if (rel == centre_rel) return csh[R + dx];
-            return win[LV][mq(rel)][0];
-        }
-    }
-
-    // Lanes beyond a side face take the boundary value of this row.
-    __device__ __forceinline__ C side_faces(C v) const
-    {
-        if (!xedge) return v;
-        if constexpr (BC == PERKS_BC_ZERO) {
-            return xout ? (C)0 : v;
-        } else {
-            const C vw = read_lane(v, lane_w);
-            const C ve = read_lane(v, lane_e);
-            return x < 0 ? vw : (x >= nx ? ve : v);
-        }
-    }
-
-    // Level LV1 = LV + 1 computes row q = i - R*LV1 from level LV's window.
-    // Window slots are written every iteration with static indices and
-    // selects (no branch around a register-array write): the slot of row q
-    // held row q - Q, which no level needs any more, so writing it when q is
-    // outside the item's range is harmless.
-    template <int U, int LV>
-    __device__ __forceinline__ void level(int i)
-    {
-        if constexpr (LV < L) {
-            constexpr int LV1 = LV + 1;
-            constexpr int REL = U - R * LV1;  // relative index of row q
-            const int q = i - R * LV1;
-            C v = (C)0;
-            if (q >= lo[LV1] && q < hi[LV1] && q < ny) {
-                C csh[Q];
-                if constexpr (!BOX) {
-                    shifts<R>(win[LV][mq(REL)][0], csh);
-                }
-                v = eval_shape<SHAPE, C, HAS_DIV>(k, kdiv, kd, [&](int dy, int dx) -> C {
-                    return cell<LV>(REL + dy, dx, csh, REL);
-                });
-                if (sr) v = Fmt<S>::qsr(v, (uint32_t)q * (uint32_t)nx + (uint32_t)x, key[LV1]);
-                else v = Fmt<S>::q(v);
-                if constexpr (LV1 == L) {
-                    if (st_ok) Fmt<S>::st(dst + (size_t)q * nx, (size_t)x, v);
-                }
-            }
-            if constexpr (LV1 < L) {
-                v = side_faces(v);
-                C row[NS];
-                if constexpr (BOX) shifts<R>(v, row);
-                else row[0] = v;
-                // Rows below the bottom face read row ny-1 (clamp) or 0 (zero).
-                const int jb = q - (ny - 1);
-#pragma unroll
-                for (int jj = 1; jj <= R; ++jj)
-#pragma unroll
-                    for (int t = 0; t < NS; ++t)
-                        row[t] = jb == jj ? (BC == PERKS_BC_ZERO ? (C)0 : win[LV1][mq(REL - jj)][t]) : row[t];
-#pragma unroll
-                for (int t = 0; t < NS; ++t) win[LV1][mq(REL)][t] = row[t];
-                // Rows above the top face read row 0 (clamp) or 0 (zero).
-#pragma unroll
-                for (int j = 1; j <= R; ++j)
-#pragma unroll
-                    for (int t = 0; t < NS; ++t)
-                        win[LV1][mq(REL - j)][t] =
-                            q == 0 ? (BC == PERKS_BC_ZERO ? (C)0 : row[t]) : win[LV1][mq(REL - j)][t];
-            }
-            level<U, LV + 1>(i);
-        }
-    }
-
-    // Iteration i (stage U = (i - i0) mod UF): level-0 row i, loaded D
-    // iterations ago, enters the window, and row i + D is requested into its
-    // in-flight slot.
-    template <int U>
-    __device__ __forceinline__ void stage(int i)
-    {
-        // The next load is issued before row i is waited for, so D loads
-        // stay in flight across the wait.
-        const Raw w = fl[U];
-        fl[U] = load(i + D);
-        const C c = arrive(i, w);
-        if constexpr (BOX) {
-            C sh[Q];
-            shifts<R>(c, sh);
-#pragma unroll
-            for (int t = 0; t < Q; ++t) win[0][mq(U)][t] = sh[t];
-        } else {
-            win[0][mq(U)][0] = c;
-        }
-        level<U, 0>(i);
-    }
-
-    template <int U>
-    __device__ __forceinline__ bool trip(int i, int iend)
-    {
-        if constexpr (U < UF) {
-            if (i > iend) return false;
-            stage<U>(i);
-            return trip<U + 1>(i + 1, iend);
-        }
-        return true;
-    }
-
-    // Rows [ys, ye) of the strip whose lane 0 is column xs0; stored columns [vx0, vx1).
-    __device__ void run(int lane, int xs0, int vx0, int vx1)
-    {
-        x = xs0 + lane;
-        xc = x < 0 ? 0 : (x >= nx ? nx - 1 : x);
-        xout = x < 0 || x >= nx;
-        xedge = xs0 < 0 || xs0 + 63 >= nx;
-        lane_w = min(max(-xs0, 0), 63);
-        lane_e = min(max(nx - 1 - xs0, 0), 63);
-        st_ok = x >= vx0 && x < vx1;
-#pragma unroll
-        for (int l = 0; l <= L; ++l) {
-            lo[l] = max(0, ys - R * (L - l));
-            // Levels below L also produce the R rows beyond the bottom face.
-            hi[l] = l == L ? ye : min(ny + R, ye + R * (L - l));
-        }
-        const int i0 = ys - R * L;
-        const int iend = ye - 1 + R * L;
-#pragma unroll
-        for (int t = 0; t < D; ++t) fl[t] = load(i0 + t);
-        for (int i = i0; trip<0>(i, iend); i += UF) {
-        }
-    }
-};
-
-// ---- two columns per lane ---------------------------------------------------------
-// Storage access to the cells of columns x0 (even) and x0 + 1 in one load or
-// store, and their rounding to the storage format.
-template <typename S>
-struct Pair2;
-template <>
-struct Pair2<float> {
-    using Raw = float2;
-    __device__ static Raw ld_raw(const float* row, size_t x0) { return *reinterpret_cast<const float2*>(row + x0); }
-    __device__ static void unpack(Raw w, float& a, float& b)
-    {
-        a = w.x;
-        b = w.y;
-    }
-    __device__ static void ld(const float* row, size_t x0, float& a, float& b)
-    {
-        const float2 v = *reinterpret_cast<const float2*>(row + x0);
-        a = v.x;
-        b = v.y;
-    }
-    __device__ static void st(float* row, size_t x0, float a, float b)
-    {
-        *reinterpret_cast<float2*>(row + x0) = make_float2(a, b);
-    }
-    __device__ static void q2(float&, float&, bool, uint32_t, uint32_t) {}
-};
-template <typename S16, int FMT>
-struct Pair16 {
-    using Raw = uint32_t;
-    __device__ static Raw ld_raw(const S16* row, size_t x0) { return *reinterpret_cast<const uint32_t*>(row + x0); }
-    __device__ static void unpack(Raw w, float& a, float& b)
-    {
-        a = widen_lo<FMT>(w);
-        b = widen_hi<FMT>(w);
-    }
-    __device__ static void ld(const S16* row, size_t x0, float& a, float& b)
-    {
-        const uint32_t w = *reinterpret_cast<const uint32_t*>(row + x0);
-        a = widen_lo<FMT>(w);
-        b = widen_hi<FMT>(w);
-    }
-    // a and b are already storage values: the conversion is exact.
-    __device__ static void st(S16* row, size_t x0, float a, float b)
-    {
-        *reinterpret_cast<uint32_t*>(row + x0) = Store16<FMT>::narrow2(a, b);
-    }
-    __device__ static void q2(float& a, float& b, bool sr, uint32_t idx0, uint32_t key)
-    {
-        if (sr) {
-            a = Fmt<S16>::qsr(a, idx0, key);
-            b = Fmt<S16>::qsr(b, idx0 + 1u, key);
-        } else {
-            const uint32_t w = Store16<FMT>::narrow2(a, b);
-            a = widen_lo<FMT>(w);
-            b = widen_hi<FMT>(w);
-        }
-    }
-};
-template <>
-struct Pair2<fmt::f16s> : Pair16<fmt::f16s, PERKS_F16> {};
-template <>
-struct Pair2<fmt::bf16s> : Pair16<fmt::bf16s, PERKS_BF16> {};
 
 // v moved by s lanes (lane i receives lane i + s), s static after unrolling.
 template <int R, typename C>
@@ -340,29 +101,134 @@ __device__ __forceinline__ void pair_shifts(C a, C b, C (&sa)[2 * R + 1], C (&sb
     }
 }
 
-// As Strip, with each lane holding two neighbouring columns (a: even x0,
-// b: x0 + 1): one load, store and set of lane shifts serves two cells.  The
-// strip is 128 columns wide and starts on an even column; the grid width must
-// be even.
-template <int SHAPE, typename S, int BC, bool HAS_DIV, int L>
-struct Strip2 {
+// ---- row access ---------------------------------------------------------------
+// Through a buffer descriptor that starts at the strip's first column inside
+// the grid and ends with the row: an offset past the end reads 0 and drops a
+// store, so lanes outside the grid (zero boundary) and lanes or rows that store
+// nothing need no select and no branch.  Raw is the register form of a loaded
+// word, unpacked when it is first used.
+template <typename S, bool PAIR>
+struct RowBuf;
+template <typename S>
+struct RowBuf<S, false> {
     using C = typename Fmt<S>::C;
+    using Raw = typename Fmt<S>::Raw;
+    __device__ static Raw ld(rsrc_t r, uint32_t off)
+    {
+        if constexpr (sizeof(S) == 2) return (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(r, (int)off, 0, 0);
+        else return buf_load(r, off, Raw{});
+    }
+    __device__ static void unpack(Raw w, C (&v)[1]) { v[0] = Fmt<S>::widen(w); }
+    __device__ static void st(rsrc_t r, uint32_t off, const C (&v)[1])
+    {
+        if constexpr (sizeof(S) == 2) {
+            S o;
+            Fmt<S>::st(&o, 0, v[0]);
+            __builtin_amdgcn_raw_buffer_store_b16(o.v, r, (int)off, 0, 0);
+        } else {
+            buf_store(r, off, v[0]);
+        }
+    }
+    __device__ static void round(C (&v)[1], bool sr, uint32_t idx, uint32_t key)
+    {
+        if (sr) v[0] = Fmt<S>::qsr(v[0], idx, key);
+        else v[0] = Fmt<S>::q(v[0]);
+    }
+};
+// Columns x (even) and x + 1 in one load or store.
+template <>
+struct RowBuf<float, true> {
+    using C = float;
+    using Raw = float2;
+    __device__ static Raw ld(rsrc_t r, uint32_t off)
+    {
+        return __builtin_bit_cast(Raw, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0));
+    }
+    __device__ static void unpack(Raw w, C (&v)[2])
+    {
+        v[0] = w.x;
+        v[1] = w.y;
+    }
+    __device__ static void st(rsrc_t r, uint32_t off, const C (&v)[2])
+    {
+        using v2i = int __attribute__((ext_vector_type(2)));
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2i, make_float2(v[0], v[1])), r, (int)off, 0, 0);
+    }
+    __device__ static void round(C (&)[2], bool, uint32_t, uint32_t) {}
+};
+template <typename S16, int FMT>
+struct RowBuf16 {
+    using C = float;
+    using Raw = uint32_t;
+    __device__ static Raw ld(rsrc_t r, uint32_t off)
+    {
+        return __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0);
+    }
+    __device__ static void unpack(Raw w, C (&v)[2])
+    {
+        v[0] = widen_lo<FMT>(w);
+        v[1] = widen_hi<FMT>(w);
+    }
+    // v holds storage values already: the conversion is exact.
+    __device__ static void st(rsrc_t r, uint32_t off, const C (&v)[2])
+    {
+        __builtin_amdgcn_raw_buffer_store_b32(Store16<FMT>::narrow2(v[0], v[1]), r, (int)off, 0, 0);
+    }
+    __device__ static void round(C (&v)[2], bool sr, uint32_t idx, uint32_t key)
+    {
+        if (sr) {
+            v[0] = Fmt<S16>::qsr(v[0], idx, key);
+            v[1] = Fmt<S16>::qsr(v[1], idx + 1u, key);
+        } else {
+            const uint32_t w = Store16<FMT>::narrow2(v[0], v[1]);
+            v[0] = widen_lo<FMT>(w);
+            v[1] = widen_hi<FMT>(w);
+        }
+    }
+};
+template <>
+struct RowBuf<fmt::f16s, true> : RowBuf16<fmt::f16s, PERKS_F16> {};
+template <>
+struct RowBuf<fmt::bf16s, true> : RowBuf16<fmt::bf16s, PERKS_BF16> {};
+
+// One work item.  PAIR: each lane holds two neighbouring columns (the strip is
+// 128 columns wide and starts on an even column; the grid width must be even),
+// so one load, store and set of lane shifts serves two cells.  EDGE: the strip
+// reaches past a side face, or the segment's rows (its ghost rows included)
+// reach row 0 or past the last one.
+//
+// A level computes a row as soon as the row it needs last arrives, without
+// asking whether the others have: the first R*l rows of a segment come out of a
+// window that does not hold their inputs yet, as values that no stored row
+// reads.  Every row also stores, where there is nothing to store to a descriptor of
+// size 0.  So away from the faces a row costs its update and some 15 scalar
+// operations, whatever the depth of the pass.  The 5-point star in FP32 has 9
+// vector operations per row and level; the form with range and face tests and
+// 64-bit addresses per row and level had some 20 scalar ones beside them, issued at
+// the same rate.
+//
+// And the loop has one way in, one back edge and the same memory operations on
+// both: the compiler's waits for the rows in flight are those of the steady
+// state.  With an exit or a conditional store between the rows it waited for
+// every operation in flight once per trip.
+template <int SHAPE, typename S, int BC, bool HAS_DIV, int L, bool PAIR, bool EDGE>
+struct Strip {
+    using C = typename Fmt<S>::C;
+    using Row = RowBuf<S, PAIR>;
+    using Raw = typename Row::Raw;
     static constexpr const ShapeDesc& SD = shape_desc<SHAPE>();
     static constexpr int R = SD.radius;
     static constexpr bool BOX = SD.is_box != 0;
-    static constexpr int Q = 2 * R + 1;
-    static constexpr int D = Q * ((8 + Q - 1) / Q);
-    static constexpr int UF = D;
-    static constexpr int NS = BOX ? Q : 1;
+    static constexpr bool ZERO = BC == PERKS_BC_ZERO;
+    static constexpr int Q = 2 * R + 1;       // rows of a level's window
+    static constexpr int D = stream_trip(R);  // level-0 rows loaded ahead: a multiple of Q
+    static constexpr int UF = D;              // rows per loop trip, so every ring slot is static
+    static constexpr int NS = BOX ? Q : 1;    // boxes keep the x shifts of a row
+    static constexpr int H = PAIR ? 2 : 1;    // columns per lane
 
     const S* src;
     S* dst;
     int nx, ny;
-    int x0;              // this lane's even column
-    bool pout, xedge;    // pair outside the grid; strip reaches past a side face
-    int lane_w, lane_e;  // lanes holding columns 0 (half a) and nx-1 (half b)
-    bool st_ok;
-    int lo[L + 1], hi[L + 1];
     int ys, ye;
     C k[kMaxGroups];
     double kd[kMaxGroups];
@@ -370,179 +236,210 @@ struct Strip2 {
     bool sr;
     uint32_t key[L + 1];
 
-    using Raw = typename Pair2<S>::Raw;
-    Raw fl[D];  // level-0 rows in flight, as loaded (row i in slot (i - i0) mod D)
-    C win[L][Q][NS][2];
+    int x;                // this lane's first column
+    bool out;             // the lane lies outside the grid
+    bool xedge;           // the strip reaches past a side face
+    int lane_w, lane_e;   // lanes holding columns 0 and nx-1 (clamped into the wave)
+    uint32_t loff, soff;  // byte offsets from the descriptors' first column: load, store
+    uint32_t span;        // bytes from that column to the row's end
+    size_t row_bytes;
+    const char* lp;       // the next row to load
+    char* sp;             // the next row to store
+    int lrow, lend;       // index of the next row to load, and of the last that is needed
 
-    static constexpr int mq(int v) { return ((v % Q) + Q) % Q; }
+    Raw fl[D];            // level-0 rows in flight (row i in slot (i - i0) mod D)
+    C win[L][Q][NS][H];   // level l's window
 
-    __device__ __forceinline__ Raw load(int q) const
+    static constexpr int mq(int a) { return ((a % Q) + Q) % Q; }
+
+    // Rows above the grid: row 0 (clamp) or nothing (zero: 0); below it, the same
+    // rule.  The rows requested past the last one needed are that one again, from
+    // the L1 (leaving them out costs a descriptor change per row: 4-6% of a pass).
+    __device__ __forceinline__ Raw next_row()
     {
-        const int qc = q < 0 ? 0 : (q >= ny ? ny - 1 : q);
-        const int xc = x0 < 0 ? 0 : (x0 > nx - 2 ? nx - 2 : x0);
-        return Pair2<S>::ld_raw(src + (size_t)qc * nx, (size_t)xc);
+        const bool in = !EDGE || !ZERO || (uint32_t)lrow < (uint32_t)ny;
+        const Raw w = Row::ld(make_rsrc(lp, in ? span : 0u), loff);
+        lp += (!EDGE || lrow >= 0) && lrow < lend ? row_bytes : 0;
+        ++lrow;
+        return w;
     }
 
-    // Row q of level 0 from its loaded word, at its first use (D rows after
-    // its load was issued): unpacked, with the boundary rule applied to pairs
-    // outside the grid.
-    __device__ __forceinline__ void arrive(int q, Raw w, C& oa, C& ob) const
+    __device__ __forceinline__ void store(bool ok, const C (&v)[H])
     {
-        C a, b;
-        Pair2<S>::unpack(w, a, b);
-        if constexpr (BC == PERKS_BC_ZERO) {
-            const bool z = q < 0 || q >= ny || pout;
-            oa = z ? (C)0 : a;
-            ob = z ? (C)0 : b;
+        Row::st(make_rsrc(sp, ok ? span : 0u), soff, v);
+        sp += row_bytes;
+    }
+
+    // sh[h][R + dx]: the value at column x + h + dx.
+    __device__ __forceinline__ static void shift_row(const C (&v)[H], C (&sh)[H][Q])
+    {
+        if constexpr (PAIR) pair_shifts<R>(v[0], v[1], sh[0], sh[1]);
+        else shifts<R>(v[0], sh[0]);
+    }
+
+    __device__ __forceinline__ void keep(int lv, int slot, const C (&v)[H])
+    {
+        if constexpr (BOX) {
+            C sh[H][Q];
+            shift_row(v, sh);
+#pragma unroll
+            for (int t = 0; t < Q; ++t)
+#pragma unroll
+                for (int h = 0; h < H; ++h) win[lv][slot][t][h] = sh[h][t];
         } else {
-            oa = x0 > nx - 2 ? b : a;  // right of the grid: column nx-1 twice
-            ob = x0 < 0 ? a : b;       // left of the grid: column 0 twice
+#pragma unroll
+            for (int h = 0; h < H; ++h) win[lv][slot][0][h] = v[h];
         }
     }
 
-    template <int LV>
-    __device__ __forceinline__ C cell(int rel, int dx, int h, const C (&csa)[Q], const C (&csb)[Q], int centre) const
+    // Lanes beyond a side face take the boundary value of their row.
+    __device__ __forceinline__ void side_faces(C (&v)[H]) const
     {
-        if constexpr (BOX) return win[LV][mq(rel)][R + dx][h];
-        else {
-            if (rel == centre) return h ? csb[R + dx] : csa[R + dx];
-            return win[LV][mq(rel)][0][h];
-        }
-    }
-
-    __device__ __forceinline__ void side_faces(C& a, C& b) const
-    {
-        if (!xedge) return;
-        if constexpr (BC == PERKS_BC_ZERO) {
-            a = pout ? (C)0 : a;
-            b = pout ? (C)0 : b;
+        if constexpr (ZERO) {
+#pragma unroll
+            for (int h = 0; h < H; ++h) v[h] = out ? (C)0 : v[h];
         } else {
-            const C vw = read_lane(a, lane_w);
-            const C ve = read_lane(b, lane_e);
-            a = x0 < 0 ? vw : (x0 > nx - 2 ? ve : a);
-            b = x0 < 0 ? vw : (x0 > nx - 2 ? ve : b);
+            const C vw = read_lane(v[0], lane_w);
+            const C ve = read_lane(v[H - 1], lane_e);
+#pragma unroll
+            for (int h = 0; h < H; ++h) v[h] = out ? (x < 0 ? vw : ve) : v[h];
         }
     }
 
+    // Level LV1 = LV + 1 computes row q = i - R*LV1 from level LV's window.  The
+    // slot it writes held row q - Q, which no level needs any more.
     template <int U, int LV>
     __device__ __forceinline__ void level(int i)
     {
         if constexpr (LV < L) {
             constexpr int LV1 = LV + 1;
-            constexpr int REL = U - R * LV1;
+            constexpr int REL = U - R * LV1;  // relative index of row q
             const int q = i - R * LV1;
-            C va = (C)0, vb = (C)0;
-            if (q >= lo[LV1] && q < hi[LV1] && q < ny) {
-                C csa[Q], csb[Q];
-                if constexpr (!BOX) {
-                    pair_shifts<R>(win[LV][mq(REL)][0][0], win[LV][mq(REL)][0][1], csa, csb);
-                }
-                va = eval_shape<SHAPE, C, HAS_DIV>(k, kdiv, kd, [&](int dy, int dx) -> C {
-                    return cell<LV>(REL + dy, dx, 0, csa, csb, REL);
-                });
-                vb = eval_shape<SHAPE, C, HAS_DIV>(k, kdiv, kd, [&](int dy, int dx) -> C {
-                    return cell<LV>(REL + dy, dx, 1, csa, csb, REL);
-                });
-                Pair2<S>::q2(va, vb, sr, (uint32_t)q * (uint32_t)nx + (uint32_t)x0, key[LV1]);
-                if constexpr (LV1 == L) {
-                    if (st_ok) Pair2<S>::st(dst + (size_t)q * nx, (size_t)x0, va, vb);
-                }
+            C sh[H][Q];
+            if constexpr (!BOX) {
+                C c[H];
+#pragma unroll
+                for (int h = 0; h < H; ++h) c[h] = win[LV][mq(REL)][0][h];
+                shift_row(c, sh);
             }
-            if constexpr (LV1 < L) {
-                side_faces(va, vb);
-                C row[NS][2];
-                if constexpr (BOX) {
-                    C sa[Q], sb[Q];
-                    pair_shifts<R>(va, vb, sa, sb);
+            C v[H];
 #pragma unroll
-                    for (int t = 0; t < Q; ++t) {
-                        row[t][0] = sa[t];
-                        row[t][1] = sb[t];
+            for (int h = 0; h < H; ++h)
+                v[h] = eval_shape<SHAPE, C, HAS_DIV>(k, kdiv, kd, [&](int dy, int dx) -> C {
+                    if constexpr (BOX) return win[LV][mq(REL + dy)][R + dx][h];
+                    else return dy == 0 ? sh[h][R + dx] : win[LV][mq(REL + dy)][0][h];
+                });
+            if constexpr (sizeof(S) == 2)
+                Row::round(v, sr, (uint32_t)q * (uint32_t)nx + (uint32_t)x, key[LV1]);
+            if constexpr (LV1 == L) {
+                store((uint32_t)(q - ys) < (uint32_t)(ye - ys), v);
+            } else {
+                if constexpr (EDGE) {
+                    if (rarely(xedge)) {
+                        keep_branch();
+                        side_faces(v);
                     }
-                } else {
-                    row[0][0] = va;
-                    row[0][1] = vb;
+                    if (rarely((uint32_t)q >= (uint32_t)ny)) {
+                        // Rows below the bottom face read row ny-1 (clamp) or 0 (zero).
+                        // (Above the top one: 0, or row 0 once it is known, below.)
+                        keep_branch();
+#pragma unroll
+                        for (int h = 0; h < H; ++h) v[h] = ZERO ? (C)0 : win[LV1][mq(REL - 1)][BOX ? R : 0][h];
+                    }
                 }
-                const int jb = q - (ny - 1);
+                keep(LV1, mq(REL), v);
+                if constexpr (EDGE && !ZERO) {
+                    if (rarely(q == 0)) {
+                        // Rows above the top face read row 0.
+                        keep_branch();
 #pragma unroll
-                for (int jj = 1; jj <= R; ++jj)
+                        for (int j = 1; j <= R; ++j)
 #pragma unroll
-                    for (int t = 0; t < NS; ++t)
+                            for (int t = 0; t < NS; ++t)
 #pragma unroll
-                        for (int h = 0; h < 2; ++h)
-                            row[t][h] = jb == jj ? (BC == PERKS_BC_ZERO ? (C)0 : win[LV1][mq(REL - jj)][t][h])
-                                                 : row[t][h];
-#pragma unroll
-                for (int t = 0; t < NS; ++t) {
-                    win[LV1][mq(REL)][t][0] = row[t][0];
-                    win[LV1][mq(REL)][t][1] = row[t][1];
+                                for (int h = 0; h < H; ++h)
+                                    win[LV1][mq(REL - j)][t][h] = win[LV1][mq(REL)][t][h];
+                    }
                 }
-#pragma unroll
-                for (int j = 1; j <= R; ++j)
-#pragma unroll
-                    for (int t = 0; t < NS; ++t)
-#pragma unroll
-                        for (int h = 0; h < 2; ++h)
-                            win[LV1][mq(REL - j)][t][h] =
-                                q == 0 ? (BC == PERKS_BC_ZERO ? (C)0 : row[t][h]) : win[LV1][mq(REL - j)][t][h];
             }
             level<U, LV + 1>(i);
         }
     }
 
+    // Iteration i (stage U = (i - i0) mod UF): level-0 row i, loaded D
+    // iterations ago, enters the window, and row i + D is requested into its
+    // in-flight slot.
     template <int U>
     __device__ __forceinline__ void stage(int i)
     {
         const Raw w = fl[U];
-        fl[U] = load(i + D);  // issued before row i is waited for
-        C a, b;
-        arrive(i, w, a, b);
-        if constexpr (BOX) {
-            C sa[Q], sb[Q];
-            pair_shifts<R>(a, b, sa, sb);
-#pragma unroll
-            for (int t = 0; t < Q; ++t) {
-                win[0][mq(U)][t][0] = sa[t];
-                win[0][mq(U)][t][1] = sb[t];
+        fl[U] = next_row();  // issued before row i is waited for
+        C v[H];
+        Row::unpack(w, v);
+        if constexpr (EDGE && PAIR && !ZERO) {
+            if (rarely(xedge)) {
+                // a pair beyond a side face loaded the edge pair: both halves take the edge column
+                keep_branch();
+                const C a = v[0], b = v[1];
+                v[0] = x > nx - 2 ? b : a;
+                v[1] = x < 0 ? a : b;
             }
-        } else {
-            win[0][mq(U)][0][0] = a;
-            win[0][mq(U)][0][1] = b;
         }
+        keep(0, mq(U), v);
         level<U, 0>(i);
     }
 
-    template <int U>
-    __device__ __forceinline__ bool trip(int i, int iend)
+    // One trip.  Rows past the segment's last are computed and not stored
+    // (segments are cut to whole trips where they can be, cut_rows in j2d.hip).
+    template <int U = 0>
+    __device__ __forceinline__ void trip(int i)
     {
         if constexpr (U < UF) {
-            if (i > iend) return false;
             stage<U>(i);
-            return trip<U + 1>(i + 1, iend);
+            // Rows are scheduled one by one: mixed, their values take up to
+            // 50% more registers.
+            __builtin_amdgcn_sched_barrier(0);
+            trip<U + 1>(i + 1);
         }
-        return true;
     }
 
-    // Strip whose lane 0 holds columns xs0, xs0+1 (xs0 even); stores columns [vx0, vx1).
-    __device__ void run(int lane, int xs0, int vx0, int vx1)
+    // Rows [ys, ye) of the strip whose lane 0 holds column xs0; stores columns [vx0, vx1).
+    __device__ __forceinline__ void run(int lane, int xs0, int vx0, int vx1)
     {
-        x0 = xs0 + 2 * lane;
-        pout = x0 < 0 || x0 > nx - 2;
-        xedge = xs0 < 0 || xs0 + 127 > nx - 1;
-        lane_w = min(max(-xs0 / 2, 0), 63);
-        lane_e = min(max((nx - 2 - xs0) / 2, 0), 63);
-        st_ok = x0 >= vx0 && x0 < vx1;
-#pragma unroll
-        for (int l = 0; l <= L; ++l) {
-            lo[l] = max(0, ys - R * (L - l));
-            hi[l] = l == L ? ye : min(ny + R, ye + R * (L - l));
-        }
+        x = xs0 + H * lane;
+        out = x < 0 || x > nx - H;
+        xedge = xs0 < 0 || xs0 + 64 * H - 1 >= nx;
+        lane_w = min(max(-xs0 / H, 0), 63);
+        lane_e = min(max((nx - H - xs0) / H, 0), 63);
+        const int xb = max(xs0, 0);  // the descriptors' first column
+        const int xc = x < 0 ? 0 : (x > nx - H ? nx - H : x);
+        loff = ZERO && out ? kOob : (uint32_t)(xc - xb) * (uint32_t)sizeof(S);
+        soff = x >= vx0 && x < vx1 ? (uint32_t)(x - xb) * (uint32_t)sizeof(S) : kOob;
+        row_bytes = (size_t)nx * sizeof(S);
+        span = (uint32_t)(min(nx - xb, 64 * H) * (int)sizeof(S));
         const int i0 = ys - R * L;
         const int iend = ye - 1 + R * L;
+        lrow = i0;
+        lend = min(iend, ny - 1);
+        lp = reinterpret_cast<const char*>(src + (size_t)max(i0, 0) * nx + xb);
+        // the row that iteration i0 stores, D rows further for the ones dropped below
+        sp = reinterpret_cast<char*>(dst + xb) + (ptrdiff_t)(i0 - R * L - D) * (ptrdiff_t)row_bytes;
 #pragma unroll
-        for (int t = 0; t < D; ++t) fl[t] = load(i0 + t);
-        for (int i = i0; trip<0>(i, iend); i += UF) {
+        for (int l = 0; l < L; ++l)
+#pragma unroll
+            for (int q = 0; q < Q; ++q)
+#pragma unroll
+                for (int t = 0; t < NS; ++t)
+#pragma unroll
+                    for (int h = 0; h < H; ++h) win[l][q][t][h] = (C)0;
+        // The rows in flight, each followed by a dropped store as in the loop.
+        const C none[H] = {};
+#pragma unroll
+        for (int t = 0; t < D; ++t) {
+            fl[t] = next_row();
+            store(false, none);
         }
+        for (int i = i0; i <= iend; i += UF) trip(i);
     }
 };
 
@@ -587,16 +484,16 @@ __global__ void __launch_bounds__(kWaves * 64) j2d_stream_kernel(J2dArgs a, KCoe
             const int vx0 = tx * VW, vx1 = min(vx0 + VW, gd.nx);
             const S* src = (const S*)((gp & 1) ? gd.b : gd.a);
             S* dst = (S*)((gp & 1) ? gd.a : gd.b);
-            auto go = [&](auto lv) {
+            const int ys = sg == 0 ? 0 : gd.seg0 + (sg - 1) * gd.seg;
+            const int ye = sg == 0 ? gd.seg0 : min(ys + gd.seg, gd.ny);
+            auto run = [&](auto lv, auto& s) {
                 constexpr int LL = decltype(lv)::value;
-                using St = std::conditional_t<PAIR, Strip2<SHAPE, S, BC, HAS_DIV, LL>, Strip<SHAPE, S, BC, HAS_DIV, LL>>;
-                St s;
                 s.src = src;
                 s.dst = dst;
                 s.nx = gd.nx;
                 s.ny = gd.ny;
-                s.ys = sg * gd.seg;
-                s.ye = min(s.ys + gd.seg, gd.ny);
+                s.ys = ys;
+                s.ye = ye;
 #pragma unroll
                 for (int g = 0; g < kMaxGroups; ++g) {
                     s.k[g] = k[g];
@@ -608,6 +505,18 @@ __global__ void __launch_bounds__(kWaves * 64) j2d_stream_kernel(J2dArgs a, KCoe
                 for (int l = 1; l <= LL; ++l)
                     s.key[l] = a.sr ? sr_key((uint32_t)(gp * a.levels + l - 1), a.seed) : 0u;
                 s.run(lane, vx0 - (PAIR ? pair_ghost(R, LL) : R * LL), vx0, vx1);
+            };
+            auto go = [&](auto lv) {
+                constexpr int LL = decltype(lv)::value;
+                constexpr int RL = R * LL;
+                const int xs0 = vx0 - (PAIR ? pair_ghost(R, LL) : RL);
+                if (xs0 < 0 || xs0 + (PAIR ? 127 : 63) >= gd.nx || ys <= RL || ye + RL > gd.ny) {
+                    Strip<SHAPE, S, BC, HAS_DIV, LL, PAIR, true> s;
+                    run(lv, s);
+                } else {
+                    Strip<SHAPE, S, BC, HAS_DIV, LL, PAIR, false> s;
+                    run(lv, s);
+                }
             };
             if (L <= 1 || LM < 2) {
                 go(std::integral_constant<int, 1>{});
