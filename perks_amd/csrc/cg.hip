@@ -80,7 +80,6 @@ namespace perks {
 namespace {
 
 constexpr int kLanes = 256;
-constexpr int kWaves = kLanes / 64;
 constexpr int kPerLane = 16;
 constexpr int kSeg = kLanes * kPerLane;
 constexpr int kMaxDiag = 16;
@@ -88,6 +87,13 @@ constexpr int kCsrChunk = 8;    // entries of a short row loaded per predicated 
 constexpr int kShortRow = 64;   // CSR rows up to this length: one lane
 constexpr int kRowChunk = 4096; // longer rows: chunks of at most this many entries, one wave each
 constexpr int kMaxWgPerCu = kCoopMaxWavesPerCu / 4;  // 256-thread workgroups
+
+// NG, the kernels' template argument: groups of kLanes threads per workgroup.  A
+// segment's 16 rows per lane are shared out to the groups in order, so NG > 1
+// runs one segment with NG times the waves.  With fewer segments than the chip
+// holds workgroups that is what shortens an iteration: at 64^3 (64 segments)
+// one group per workgroup leaves 4 waves on each of 64 CUs, and an iteration is
+// the latency of 16 rows one after the other.
 
 // Matrix formats the kernel is built for.  DIA7 is the 7-diagonal form with
 // the diagonal count fixed at compile time (every load of a row issued at once).
@@ -159,8 +165,18 @@ struct CgArgs {
 };
 
 // ---- reductions ----------------------------------------------------------
-// Folds the 256 per-lane values of a workgroup pairwise with strides
-// 128, 64, ..., 1 (v[l] += v[l + s]); returns the result in every lane.
+__device__ __forceinline__ int lane256() { return (int)threadIdx.x & (kLanes - 1); }
+// Rows of a segment per lane and thread, and the first of this thread's.
+template <int NG>
+constexpr int kPerThread = kPerLane / NG;
+template <int NG>
+__device__ __forceinline__ int first_row()
+{
+    return NG == 1 ? 0 : ((int)threadIdx.x / kLanes) * kPerThread<NG>;
+}
+
+// Folds the 256 per-lane values of a workgroup of one group pairwise with
+// strides 128, 64, ..., 1 (v[l] += v[l + s]); returns the result in every lane.
 __device__ __forceinline__ double fold256(double v, double* lds)
 {
     const int t = threadIdx.x;
@@ -181,13 +197,89 @@ __device__ __forceinline__ double fold256(double v, double* lds)
     return r;
 }
 
+// The same fold by one wave whose lane l holds lanes l, l+64, l+128 and l+192:
+// the first two strides stay inside a lane.  The result is in lane 0.
+__device__ __forceinline__ double fold_wave(const double (&c)[4])
+{
+    double u = (c[0] + c[2]) + (c[1] + c[3]);
+#pragma unroll
+    for (int s = 32; s >= 1; s >>= 1) u = u + __shfl_down(u, s, 64);
+    return u;
+}
+
+// Sum of a segment's products, each lane's 16 in row order from zero and then
+// the fold.  One group: every thread adds its lane's products itself, and the
+// workgroup folds.  More: the products of all groups but the last go to LDS, the
+// last group adds them and then its own, lane by lane, and one wave folds the
+// lanes; the sum is in thread 0 only.
+template <int NG>
+constexpr int kSumDoubles = NG == 1 ? kLanes : (kPerLane - kPerThread<NG> + 1) * kLanes;
+template <int NG>
+struct SegSum {
+    double* lds;  // kSumDoubles<NG>
+    double acc = 0.0;
+    double own[NG == 1 ? 1 : kPerThread<NG>];  // this thread's products (several groups)
+    __device__ __forceinline__ explicit SegSum(double* l) : lds(l)
+    {
+        if (NG > 1) __syncthreads();  // the last sum's values have been read
+    }
+    // Product of row kk of this lane; valid: the row takes part.
+    __device__ __forceinline__ void add(int kk, double v, bool valid = true)
+    {
+        if constexpr (NG == 1) {
+            if (valid) acc = acc + v;
+        } else {
+            const double x = valid ? v : 0.0;  // s + 0 is s: no sum here is -0
+            if (kk < kPerLane - kPerThread<NG>) lds[kk * kLanes + lane256()] = x;
+#pragma unroll
+            for (int j = 0; j < kPerThread<NG>; ++j) own[j] = (kk & (kPerThread<NG> - 1)) == j ? x : own[j];
+        }
+    }
+    __device__ __forceinline__ double finish()
+    {
+        if constexpr (NG == 1) {
+            return fold256(acc, lds);
+        } else {
+            constexpr int N = kPerLane - kPerThread<NG>;
+            double* const sums = lds + N * kLanes;
+            __syncthreads();
+            if ((int)threadIdx.x >= (NG - 1) * kLanes) {
+#pragma unroll
+                for (int kk = 0; kk < N; ++kk) acc = acc + lds[kk * kLanes + lane256()];
+#pragma unroll
+                for (int j = 0; j < kPerThread<NG>; ++j) acc = acc + own[j];
+                sums[lane256()] = acc;
+            }
+            __syncthreads();
+            if (threadIdx.x >= 64) return 0.0;
+            const double c[4] = {sums[threadIdx.x], sums[threadIdx.x + 64], sums[threadIdx.x + 128],
+                                 sums[threadIdx.x + 192]};
+            return fold_wave(c);
+        }
+    }
+};
+
 // Sum of the segment partials in the fixed order: lane l sums partials
-// l, l+256, ... in order, then the 256-lane fold.
+// l, l+256, ... in order, then the 256-lane fold.  With several groups there are
+// few partials, and every wave sums them by itself.
+template <int NG>
 __device__ __forceinline__ double reduce_parts(const double* part, int nseg, double* lds)
 {
-    double acc = 0.0;
-    for (int j = threadIdx.x; j < nseg; j += kLanes) acc = acc + part[j];
-    return fold256(acc, lds);
+    if constexpr (NG == 1) {
+        double acc = 0.0;
+        for (int j = threadIdx.x; j < nseg; j += kLanes) acc = acc + part[j];
+        return fold256(acc, lds);
+    } else {
+        double c[4] = {0.0, 0.0, 0.0, 0.0};
+        for (int j0 = 0; j0 < nseg; j0 += kLanes)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int i = j0 + 64 * j + ((int)threadIdx.x & 63);
+                const double v = i < nseg ? part[i] : 0.0;
+                c[j] = c[j] + v;
+            }
+        return __shfl(fold_wave(c), 0, 64);
+    }
 }
 
 template <typename V>
@@ -308,7 +400,7 @@ __device__ __forceinline__ void vput_at(const Lds<V>& c, int v, int u, int lane,
 template <bool CACHED = true, typename V>
 __device__ __forceinline__ V vget(const Lds<V>& c, int v, int u, const V* hbm, int i)
 {
-    if (CACHED && u < c.units[v]) return c.vec[v][u * kLanes + threadIdx.x];
+    if (CACHED && u < c.units[v]) return c.vec[v][u * kLanes + lane256()];
     return hbm[i];
 }
 // Stores entry i: into LDS when cached (and to HBM too when other workgroups
@@ -317,7 +409,7 @@ template <bool CACHED = true, typename V>
 __device__ __forceinline__ void vput(const Lds<V>& c, int v, int u, V* hbm, int i, V val, bool shared)
 {
     if (CACHED && u < c.units[v]) {
-        c.vec[v][u * kLanes + threadIdx.x] = val;
+        c.vec[v][u * kLanes + lane256()] = val;
         if (shared) hbm[i] = val;
     } else {
         hbm[i] = val;
@@ -512,10 +604,11 @@ __device__ __forceinline__ bool seg_cached(const CgArgs<V>& a, const Lds<V>& c, 
 }
 
 // Every chunk of every long row, one wave per chunk across the grid.
-template <typename V, class Op>
+template <int NG, typename V, class Op>
 __device__ __forceinline__ void long_chunks(const CgArgs<V>& a, const Lds<V>& c, const Op& op)
 {
     const int wave = threadIdx.x >> 6;
+    constexpr int kWaves = NG * kLanes / 64;
     for (int ci = blockIdx.x * kWaves + wave; ci < a.nchunk; ci += gridDim.x * kWaves) {
         const int j = a.lcj[ci];
         const int row = a.lrow[j];
@@ -539,16 +632,20 @@ __device__ __forceinline__ V long_value(const CgArgs<V>& a, int j)
 // r = b + (-1) * A x (r = b when x is zero); partials of r.r and b.b.  Also
 // loads the cached units of x.  Segments holding long rows get their
 // partials in fix_initial.
-template <typename V, int FMT>
+template <typename V, int FMT, int NG>
 __device__ void phase_initial(const CgArgs<V>& a, const Lds<V>& c, int me, int kb, bool fill, double* lds)
 {
-    const int t = threadIdx.x;
+    const int t = lane256();
     const OpVec<V> op{a.x};
     for_owned(a, c.slots, [&](int s, int q) {
-        double rr = 0.0, bb = 0.0;
+        double prr = 0.0, pbb = 0.0;
         int anyl = 0;
         auto rows = [&](auto irr) {
-            for (int kk = 0; kk < kPerLane; ++kk) {
+            SegSum<NG> rr(lds);
+            double bb[NG == 1 ? 1 : kPerThread<NG>] = {};  // one group: the lane's sum; else its products
+#pragma unroll NG == 1 ? 1 : 4
+            for (int k = 0; k < kPerThread<NG>; ++k) {
+                const int kk = first_row<NG>() + k;
                 const int i = s * kSeg + kk * kLanes + t;
                 const int u = q * kPerLane + kk;
                 const bool valid = i < a.n;
@@ -559,29 +656,41 @@ __device__ void phase_initial(const CgArgs<V>& a, const Lds<V>& c, int me, int k
                                                                         lng);
                 if (valid) {
                     if (u < c.units[VC_X]) c.vec[VC_X][u * kLanes + t] = a.x[i];
-                    if (!lng) {
-                        const V bi = a.b[i];
-                        const V ri = a.x_is_zero ? bi : bi + (V)(-1) * ax;
-                        vput<true>(c, VC_R, u, a.r, i, ri, true);
-                        rr = rr + prod_d(ri, ri);
-                        bb = bb + prod_d(bi, bi);
-                    }
+                }
+                V ri = (V)0, bi = (V)0;
+                if (valid && !lng) {
+                    bi = a.b[i];
+                    ri = a.x_is_zero ? bi : bi + (V)(-1) * ax;
+                    vput<true>(c, VC_R, u, a.r, i, ri, true);
+                }
+                rr.add(kk, prod_d(ri, ri), valid && !lng);
+                if constexpr (NG == 1) {
+                    if (valid && !lng) bb[0] = bb[0] + prod_d(bi, bi);
+                } else {
+                    bb[k] = prod_d(bi, bi);
                 }
                 anyl |= lng ? 1 : 0;
+            }
+            prr = rr.finish();
+            if constexpr (NG == 1) {
+                pbb = fold256(bb[0], lds);
+            } else {
+                SegSum<NG> sum(lds);
+#pragma unroll
+                for (int k = 0; k < kPerThread<NG>; ++k) sum.add(first_row<NG>() + k, bb[k]);
+                pbb = sum.finish();
             }
         };
         if (FMT == FMT_CSR && a.seg_irr[s]) rows(std::true_type{});
         else rows(std::false_type{});
-        const double prr = fold256(rr, lds);
-        const double pbb = fold256(bb, lds);
         const int any = __syncthreads_or(anyl);
-        if (t == 0 && !any) {
+        if (threadIdx.x == 0 && !any) {
             a.part_a[s] = prr;
             a.part_b[s] = pbb;
         }
     });
     if constexpr (FMT == FMT_CSR)
-        if (!a.x_is_zero) long_chunks(a, c, op);
+        if (!a.x_is_zero) long_chunks<NG>(a, c, op);
 }
 
 // After a grid barrier: the long rows of this workgroup's segments (each by
@@ -596,7 +705,7 @@ __device__ __forceinline__ void fix_long_rows(const CgArgs<V>& a, lds_ptr<const 
     int q0 = 0;  // index of the slot's first segment among the workgroup's own
     for (int k = 0; k < a.rounds; ++k) {
         const int s0 = slots[4 * k], s1 = slots[4 * k + 1];
-        for (int j = slots[4 * k + 2] + (int)threadIdx.x; j < slots[4 * k + 3]; j += kLanes) {
+        for (int j = slots[4 * k + 2] + (int)threadIdx.x; j < slots[4 * k + 3]; j += (int)blockDim.x) {
             const int row = a.lrow[j];
             const int s = row / kSeg;
             const int local = row - s * kSeg;
@@ -610,7 +719,7 @@ __device__ __forceinline__ void fix_long_rows(const CgArgs<V>& a, lds_ptr<const 
     });
 }
 
-template <typename V, int FMT>
+template <typename V, int FMT, int NG>
 __device__ void fix_initial(const CgArgs<V>& a, const Lds<V>& c, int me, double* lds)
 {
     fix_long_rows(
@@ -621,18 +730,22 @@ __device__ void fix_initial(const CgArgs<V>& a, const Lds<V>& c, int me, double*
             vput_at(c, VC_R, u, lane, a.r, row, ri, true);
         },
         [&](int s, int q) {
-            double rr = 0.0, bb = 0.0;
-            for (int kk = 0; kk < kPerLane; ++kk) {
-                const int i = s * kSeg + kk * kLanes + threadIdx.x;
-                if (i < a.n) {
-                    const V ri = vget(c, VC_R, q * kPerLane + kk, a.r, i);
-                    const V bi = a.b[i];
-                    rr = rr + prod_d(ri, ri);
-                    bb = bb + prod_d(bi, bi);
-                }
+            SegSum<NG> rr(lds);
+            for (int k = 0; k < kPerThread<NG>; ++k) {
+                const int kk = first_row<NG>() + k;
+                const int i = s * kSeg + kk * kLanes + lane256();
+                const V ri = i < a.n ? vget(c, VC_R, q * kPerLane + kk, a.r, i) : (V)0;
+                rr.add(kk, prod_d(ri, ri), i < a.n);
             }
-            const double prr = fold256(rr, lds);
-            const double pbb = fold256(bb, lds);
+            const double prr = rr.finish();
+            SegSum<NG> bb(lds);
+            for (int k = 0; k < kPerThread<NG>; ++k) {
+                const int kk = first_row<NG>() + k;
+                const int i = s * kSeg + kk * kLanes + lane256();
+                const V bi = i < a.n ? a.b[i] : (V)0;
+                bb.add(kk, prod_d(bi, bi), i < a.n);
+            }
+            const double pbb = bb.finish();
             if (threadIdx.x == 0) {
                 a.part_a[s] = prr;
                 a.part_b[s] = pbb;
@@ -642,19 +755,20 @@ __device__ void fix_initial(const CgArgs<V>& a, const Lds<V>& c, int me, double*
 
 // Phase 1 of an iteration: p = r + beta*p (stored into pnew), Ap = A p,
 // partials of p.Ap into part_a.
-template <typename V, int FMT, bool FIRST>
+template <typename V, int FMT, int NG, bool FIRST>
 __device__ void phase_spmv(const CgArgs<V>& a, const Lds<V>& c, int me, int kb, const V* pold, V* pnew, V beta,
                            bool fill, double* lds)
 {
-    const int t = threadIdx.x;
+    const int t = lane256();
     const OpP<V, FIRST> op{a.r, pold, beta};
     for_owned(a, c.slots, [&](int s, int q) {
-        double acc = 0.0;
+        SegSum<NG> sum(lds);
         int anyl = 0;
         auto rows = [&](auto irr, auto cached) {
             constexpr bool C = decltype(cached)::value;
 #pragma unroll 2
-            for (int kk = 0; kk < kPerLane; ++kk) {
+            for (int k = 0; k < kPerThread<NG>; ++k) {
+                const int kk = first_row<NG>() + k;
                 const int i = s * kSeg + kk * kLanes + t;
                 const int u = q * kPerLane + kk;
                 const bool valid = i < a.n;
@@ -668,11 +782,9 @@ __device__ void phase_spmv(const CgArgs<V>& a, const Lds<V>& c, int me, int kb, 
                     row_value<V, FMT, decltype(irr)::value, C>(a, c, kb, i, valid, u * kLanes + t, fill, op, lng);
                 if (valid) {
                     vput<C>(c, VC_P, u, pnew, i, pi, true);
-                    if (!lng) {
-                        vput<C>(c, VC_AP, u, a.ap, i, api, false);
-                        acc = acc + prod_d(pi, api);
-                    }
+                    if (!lng) vput<C>(c, VC_AP, u, a.ap, i, api, false);
                 }
+                sum.add(kk, prod_d(pi, api), valid && !lng);
                 anyl |= lng ? 1 : 0;
             }
         };
@@ -684,50 +796,55 @@ __device__ void phase_spmv(const CgArgs<V>& a, const Lds<V>& c, int me, int kb, 
             if (cv) rows(std::false_type{}, std::true_type{});
             else rows(std::false_type{}, std::false_type{});
         }
-        const double ps = fold256(acc, lds);
+        const double ps = sum.finish();
         if constexpr (FMT == FMT_CSR) {
             const int any = __syncthreads_or(anyl);
-            if (t == 0 && !any) a.part_a[s] = ps;
+            if (threadIdx.x == 0 && !any) a.part_a[s] = ps;
         } else {
-            if (t == 0) a.part_a[s] = ps;
+            if (threadIdx.x == 0) a.part_a[s] = ps;
         }
     });
-    if constexpr (FMT == FMT_CSR) long_chunks(a, c, op);
+    if constexpr (FMT == FMT_CSR) long_chunks<NG>(a, c, op);
 }
 
-template <typename V, int FMT>
+template <typename V, int FMT, int NG>
 __device__ void fix_spmv(const CgArgs<V>& a, const Lds<V>& c, int me, const V* pnew, double* lds)
 {
     fix_long_rows(
         a, c.slots,
         [&](int j, int row, int u, int lane) { vput_at(c, VC_AP, u, lane, a.ap, row, long_value(a, j), false); },
         [&](int s, int q) {
-            double acc = 0.0;
-            for (int kk = 0; kk < kPerLane; ++kk) {
-                const int i = s * kSeg + kk * kLanes + threadIdx.x;
+            SegSum<NG> sum(lds);
+            for (int k = 0; k < kPerThread<NG>; ++k) {
+                const int kk = first_row<NG>() + k;
+                const int i = s * kSeg + kk * kLanes + lane256();
+                double v = 0.0;
                 if (i < a.n) {
                     const int u = q * kPerLane + kk;
-                    acc = acc + prod_d(vget(c, VC_P, u, pnew, i), vget(c, VC_AP, u, a.ap, i));
+                    v = prod_d(vget(c, VC_P, u, pnew, i), vget(c, VC_AP, u, a.ap, i));
                 }
+                sum.add(kk, v, i < a.n);
             }
-            const double ps = fold256(acc, lds);
+            const double ps = sum.finish();
             if (threadIdx.x == 0) a.part_a[s] = ps;
         });
 }
 
 // Phase 2: x = alpha*p + x ; r = (-alpha)*Ap + r ; partials of r.r into part_b.
-template <typename V, int FMT>
+template <typename V, int FMT, int NG>
 __device__ void phase_update(const CgArgs<V>& a, const Lds<V>& c, int me, const V* pnew, V alpha, double* lds)
 {
-    const int t = threadIdx.x;
+    const int t = lane256();
     const V na = -alpha;
     for_owned(a, c.slots, [&](int s, int q) {
-        double acc = 0.0;
+        SegSum<NG> sum(lds);
         auto rows = [&](auto cached) {
             constexpr bool C = decltype(cached)::value;
 #pragma unroll 4
-            for (int kk = 0; kk < kPerLane; ++kk) {
+            for (int k = 0; k < kPerThread<NG>; ++k) {
+                const int kk = first_row<NG>() + k;
                 const int i = s * kSeg + kk * kLanes + t;
+                double v = 0.0;
                 if (i < a.n) {
                     const int u = q * kPerLane + kk;
                     const V pi = vget<C>(c, VC_P, u, pnew, i);
@@ -735,21 +852,22 @@ __device__ void phase_update(const CgArgs<V>& a, const Lds<V>& c, int me, const 
                     vput<C>(c, VC_X, u, a.x, i, xi, false);
                     const V ri = na * vget<C>(c, VC_AP, u, a.ap, i) + vget<C>(c, VC_R, u, a.r, i);
                     vput<C>(c, VC_R, u, a.r, i, ri, true);
-                    acc = acc + prod_d(ri, ri);
+                    v = prod_d(ri, ri);
                 }
+                sum.add(kk, v, i < a.n);
             }
         };
         if (q * kPerLane < c.vmax) rows(std::true_type{});
         else rows(std::false_type{});
-        const double ps = fold256(acc, lds);
-        if (t == 0) a.part_b[s] = ps;
+        const double ps = sum.finish();
+        if (threadIdx.x == 0) a.part_b[s] = ps;
     });
 }
 
-template <typename V, int FMT>
-__global__ void __launch_bounds__(kLanes) cg_persistent_kernel(CgArgs<V> a)
+template <typename V, int FMT, int NG>
+__global__ void __launch_bounds__(NG * kLanes) cg_persistent_kernel(CgArgs<V> a)
 {
-    __shared__ double lds[kLanes];
+    __shared__ double lds[kSumDoubles<NG>];
     extern __shared__ __align__(16) unsigned char cg_dyn[];
     const int t = threadIdx.x;
     const int G = gridDim.x;
@@ -759,7 +877,7 @@ __global__ void __launch_bounds__(kLanes) cg_persistent_kernel(CgArgs<V> a)
     {
         // the slot table: round k's slot is me + k * G
         lds_ptr<int> tab = reinterpret_cast<lds_ptr<int>>(dyn);
-        for (int k = t; k < a.rounds; k += kLanes) {
+        for (int k = t; k < a.rounds; k += NG * kLanes) {
             const int s0 = slot_begin<V, FMT>(a, me + k * G, G * a.rounds);
             const int s1 = slot_begin<V, FMT>(a, me + k * G + 1, G * a.rounds);
             tab[4 * k] = s0;
@@ -775,15 +893,15 @@ __global__ void __launch_bounds__(kLanes) cg_persistent_kernel(CgArgs<V> a)
     const bool has_long = FMT == FMT_CSR && a.nlong > 0;
 
     // ---- r = b + (-1) * A x ; partials of r.r and b.b ----
-    phase_initial<V, FMT>(a, c, me, kb, true, lds);
+    phase_initial<V, FMT, NG>(a, c, me, kb, true, lds);
     bool fill = a.x_is_zero != 0;  // the first SpMV fills the matrix cache
     if (!grid_sync(a.sync, G, a.timeout, true)) return;
     if (has_long && !a.x_is_zero) {
-        fix_initial<V, FMT>(a, c, me, lds);
+        fix_initial<V, FMT, NG>(a, c, me, lds);
         if (!grid_sync(a.sync, G, a.timeout, false)) return;
     }
-    double r1 = reduce_parts(a.part_a, a.nseg, lds);
-    const double bbv = reduce_parts(a.part_b, a.nseg, lds);
+    double r1 = reduce_parts<NG>(a.part_a, a.nseg, lds);
+    const double bbv = reduce_parts<NG>(a.part_b, a.nseg, lds);
     const double thr = a.relative ? a.tol2 * bbv : a.tol2;
     if (me == 0 && t == 0) {
         if (a.hist && a.hist_cap > 0) a.hist[0] = r1;
@@ -797,21 +915,21 @@ __global__ void __launch_bounds__(kLanes) cg_persistent_kernel(CgArgs<V> a)
     V* pnew = a.p1;
     while ((a.static_iter || !(r1 < thr)) && k <= a.max_iter) {
         // ---- p = r + beta*p ; Ap = A p ; partials of p.Ap ----
-        if (k == 1) phase_spmv<V, FMT, true>(a, c, me, kb, pold, pnew, (V)0, fill, lds);
-        else phase_spmv<V, FMT, false>(a, c, me, kb, pold, pnew, (V)(r1 / r0), fill, lds);
+        if (k == 1) phase_spmv<V, FMT, NG, true>(a, c, me, kb, pold, pnew, (V)0, fill, lds);
+        else phase_spmv<V, FMT, NG, false>(a, c, me, kb, pold, pnew, (V)(r1 / r0), fill, lds);
         fill = false;
         if (!grid_sync(a.sync, G, a.timeout, false)) return;
         if (has_long) {
-            fix_spmv<V, FMT>(a, c, me, pnew, lds);
+            fix_spmv<V, FMT, NG>(a, c, me, pnew, lds);
             if (!grid_sync(a.sync, G, a.timeout, false)) return;
         }
-        const double pap = reduce_parts(a.part_a, a.nseg, lds);
+        const double pap = reduce_parts<NG>(a.part_a, a.nseg, lds);
         const double alpha_d = r1 / pap;
         // ---- x = alpha*p + x ; r = (-alpha)*Ap + r ; partials of r.r ----
-        phase_update<V, FMT>(a, c, me, pnew, (V)alpha_d, lds);
+        phase_update<V, FMT, NG>(a, c, me, pnew, (V)alpha_d, lds);
         if (!grid_sync(a.sync, G, a.timeout, false)) return;
         r0 = r1;
-        r1 = reduce_parts(a.part_b, a.nseg, lds);
+        r1 = reduce_parts<NG>(a.part_b, a.nseg, lds);
         if (me == 0 && t == 0 && a.hist && k < a.hist_cap) a.hist[k] = r1;
         ++k;
         V* tmp = pold;
@@ -820,11 +938,13 @@ __global__ void __launch_bounds__(kLanes) cg_persistent_kernel(CgArgs<V> a)
     }
     // ---- the cached units of x go back to HBM ----
     if (c.units[VC_X] > 0) {
+        const int l = lane256();
         for_owned(a, c.slots, [&](int s, int q) {
-            for (int kk = 0; kk < kPerLane; ++kk) {
+            for (int k = 0; k < kPerThread<NG>; ++k) {
+                const int kk = first_row<NG>() + k;
                 const int u = q * kPerLane + kk;
-                const int i = s * kSeg + kk * kLanes + t;
-                if (u < c.units[VC_X] && i < a.n) a.x[i] = c.vec[VC_X][u * kLanes + t];
+                const int i = s * kSeg + kk * kLanes + l;
+                if (u < c.units[VC_X] && i < a.n) a.x[i] = c.vec[VC_X][u * kLanes + l];
             }
         });
     }
@@ -1010,10 +1130,18 @@ int prepare_long_rows(const int32_t* d_rowptr, int n, CgScratch& S, hipStream_t 
 
 // ---- launch planning ---------------------------------------------------------
 template <typename V, int FMT>
-const void* kernel_ptr()
+const void* kernel_ptr(int groups)
 {
-    return reinterpret_cast<const void*>(&cg_persistent_kernel<V, FMT>);
+    switch (groups) {
+    case 4: return reinterpret_cast<const void*>(&cg_persistent_kernel<V, FMT, 4>);
+    case 2: return reinterpret_cast<const void*>(&cg_persistent_kernel<V, FMT, 2>);
+    default: return reinterpret_cast<const void*>(&cg_persistent_kernel<V, FMT, 1>);
+    }
 }
+
+// Groups per workgroup: as many as keep every segment in a workgroup of its own
+// with at most kMaxWgPerCu groups per CU.
+int groups_for(int nseg, int cus) { return nseg <= cus ? 4 : (nseg <= 2 * cus ? 2 : 1); }
 
 // The grid and the workgroups' LDS caches.  The grid is CUs x occupancy (at
 // most kMaxWgPerCu per CU, at most one workgroup per segment).  A workgroup
@@ -1038,19 +1166,20 @@ static long long lds_share(long long per_wg)
 }
 
 template <typename V, int FMT>
-int plan_launch(const CgArgs<V>& a, const perks_cg_opts* o, int* grid, CgCache* cache)
+int plan_launch(const CgArgs<V>& a, const perks_cg_opts* o, int* grid, int* groups, CgCache* cache)
 {
-    const void* fn = kernel_ptr<V, FMT>();
     perks_device_caps caps;
     int rc = device_caps_cached(&caps);
     if (rc != PERKS_OK) return rc;
+    const int ng = groups_for(a.nseg, caps.cu_count);
+    const void* fn = kernel_ptr<V, FMT>(ng);
     int occ = 0;
-    PERKS_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, kLanes, 0));
+    PERKS_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, ng * kLanes, 0));
     if (occ <= 0) return PERKS_ERR_NOT_LAUNCHABLE;
     if (o->blkpsm > 0 && o->blkpsm < occ) occ = o->blkpsm;
     // At most half the wave slots: 4 workgroups of 4 waves per CU keep enough
     // loads in flight, and the cooperative grid never needs every slot free.
-    if (occ > kMaxWgPerCu) occ = kMaxWgPerCu;
+    if (occ > kMaxWgPerCu / ng) occ = kMaxWgPerCu / ng;
     int G = caps.cu_count * occ;
     if (G > a.nseg) G = a.nseg > 0 ? a.nseg : 1;
     const int wpc = (G + caps.cu_count - 1) / caps.cu_count;
@@ -1089,13 +1218,14 @@ int plan_launch(const CgArgs<V>& a, const perks_cg_opts* o, int* grid, CgCache* 
             budget = (lds_share(65536) - (long long)fa.sharedSizeBytes - table) / 256 * 256;
             continue;
         }
-        PERKS_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ2, fn, kLanes, (size_t)c.bytes));
+        PERKS_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ2, fn, ng * kLanes, (size_t)c.bytes));
         if (occ2 >= wpc) break;
         budget -= 4096;
     }
     if (c.bytes == 0) c.bytes = (int)table;
     c.table = (int)table;
     *grid = G;
+    *groups = ng;
     *cache = c;
     return PERKS_OK;
 }
@@ -1104,16 +1234,16 @@ template <typename V, int FMT>
 int launch_cg(CgArgs<V>& a, GridSync* gs, hipStream_t stream, const perks_cg_opts* o, int* grid_out,
               CgCache* cache_out)
 {
-    int G = 0;
+    int G = 0, ng = 1;
     CgCache c;
-    const int rc = plan_launch<V, FMT>(a, o, &G, &c);
+    const int rc = plan_launch<V, FMT>(a, o, &G, &ng, &c);
     if (rc != PERKS_OK) return rc;
     a.cache = c;
     a.rounds = (a.nseg + G - 1) / G;
     a.sync = gs;
     a.timeout = grid_sync_timeout();
     void* args[] = {&a};
-    PERKS_HIP_TRY(launch_persistent(kernel_ptr<V, FMT>(), dim3(G), dim3(kLanes), args, (size_t)c.bytes, stream));
+    PERKS_HIP_TRY(launch_persistent(kernel_ptr<V, FMT>(ng), dim3(G), dim3(ng * kLanes), args, (size_t)c.bytes, stream));
     if (grid_out) *grid_out = G;
     if (cache_out) *cache_out = c;
     return PERKS_OK;
