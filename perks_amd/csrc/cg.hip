@@ -124,6 +124,7 @@ struct CgArgs {
     const int32_t* rowptr;
     const int32_t* col;
     const V* val;
+    long long nnz;
     int ndiag;
     int32_t offs[kMaxDiag];
     // vectors
@@ -302,7 +303,7 @@ __device__ __forceinline__ long long seg_cost(const CgArgs<V>& a, int s)
 
 // First segment of slot c of S: the first whose cost reaches c/S of the total.
 template <typename V, int FMT>
-__device__ int slot_begin(const CgArgs<V>& a, int c, int S)
+__device__ __forceinline__ int slot_begin(const CgArgs<V>& a, int c, int S)
 {
     if (c <= 0) return 0;
     if (c >= S) return a.nseg;
@@ -331,7 +332,7 @@ __device__ __forceinline__ void for_owned(const CgArgs<V>& a, lds_ptr<const int>
 
 // First long row at or after row `row` (index into lrow).
 template <typename V>
-__device__ int long_begin(const CgArgs<V>& a, long long row)
+__device__ __forceinline__ int long_begin(const CgArgs<V>& a, long long row)
 {
     int lo = 0, hi = a.nlong;
     while (lo < hi) {
@@ -432,12 +433,49 @@ struct OpP {
 };
 
 // ---- CSR rows ----------------------------------------------------------------
+// Eight consecutive columns or values from element-aligned memory, in 16-byte
+// loads.
+__device__ __forceinline__ void load8(const int32_t* p, int (&o)[8])
+{
+    typedef int v4 __attribute__((ext_vector_type(4), aligned(4)));
+    const v4 a = *reinterpret_cast<const v4*>(p), b = *reinterpret_cast<const v4*>(p + 4);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        o[u] = a[u];
+        o[u + 4] = b[u];
+    }
+}
+__device__ __forceinline__ void load8(const float* p, float (&o)[8])
+{
+    typedef float v4 __attribute__((ext_vector_type(4), aligned(4)));
+    const v4 a = *reinterpret_cast<const v4*>(p), b = *reinterpret_cast<const v4*>(p + 4);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        o[u] = a[u];
+        o[u + 4] = b[u];
+    }
+}
+__device__ __forceinline__ void load8(const double* p, double (&o)[8])
+{
+    typedef double v2 __attribute__((ext_vector_type(2), aligned(8)));
+#pragma unroll
+    for (int u = 0; u < 8; u += 2) {
+        const v2 a = *reinterpret_cast<const v2*>(p + u);
+        o[u] = a[0];
+        o[u + 1] = a[1];
+    }
+}
+
 // A short row [k0, k1) by its own lane, in storage order from zero.  All
 // loads of a step are issued together (out-of-row slots read the row's first
 // entry and the sum keeps its value through a select).  The entries come from
 // `cols`/`vals` (HBM, or the workgroup's cached prefix in LDS); with fill,
 // what is loaded is also stored into the prefix (entries from kb).
-template <typename V, class Op, class CP, class VP>
+// WIDE: eight entries from k2 on may be read whatever the row's length (they
+// end before the matrix does): in 16-byte loads, six instead of sixteen.  Rows
+// of a lane lie some 56 bytes from the next lane's, so an instruction's cost is
+// the lines it touches, not its bytes.
+template <bool WIDE, typename V, class Op, class CP, class VP>
 __device__ __forceinline__ V csr_short_from(CP cols, VP vals, int off, int k0, int k1, const Lds<V>& c, int kb,
                                             bool fill, const Op& op)
 {
@@ -445,11 +483,20 @@ __device__ __forceinline__ V csr_short_from(CP cols, VP vals, int off, int k0, i
     for (int k2 = k0; k2 < k1; k2 += kCsrChunk) {
         int cj[kCsrChunk];
         V cv[kCsrChunk];
+        if constexpr (WIDE) {
+            static_assert(kCsrChunk == 8);
+            load8(cols + (k2 - off), cj);
+            load8(vals + (k2 - off), cv);
+            // past the row: its first column, which is at hand
 #pragma unroll
-        for (int u = 0; u < kCsrChunk; ++u) {
-            const int k = (k2 + u < k1) ? k2 + u : k0;
-            cj[u] = cols[k - off];
-            cv[u] = vals[k - off];
+            for (int u = 1; u < kCsrChunk; ++u) cj[u] = k2 + u < k1 ? cj[u] : cj[0];
+        } else {
+#pragma unroll
+            for (int u = 0; u < kCsrChunk; ++u) {
+                const int k = (k2 + u < k1) ? k2 + u : k0;
+                cj[u] = cols[k - off];
+                cv[u] = vals[k - off];
+            }
         }
         if (fill) {
 #pragma unroll
@@ -473,8 +520,8 @@ template <typename V, class Op>
 __device__ __forceinline__ V csr_short(const CgArgs<V>& a, const Lds<V>& c, int kb, int k0, int k1,
                                        bool cached, bool fill, const Op& op)
 {
-    if (cached && !fill) return csr_short_from<V>(c.mcol, c.mval, (int)kb, k0, k1, c, kb, false, op);
-    return csr_short_from<V>(a.col, a.val, 0, k0, k1, c, kb, cached && fill, op);
+    if (cached && !fill) return csr_short_from<false, V>(c.mcol, c.mval, (int)kb, k0, k1, c, kb, false, op);
+    return csr_short_from<false, V>(a.col, a.val, 0, k0, k1, c, kb, cached && fill, op);
 }
 
 // Entries [k0, k1) (at most kRowChunk) by a whole wave: lane l sums entries
@@ -547,7 +594,10 @@ __device__ __forceinline__ V csr_row(const CgArgs<V>& a, const Lds<V>& c, int kb
 // lr: the row's index among the workgroup's rows (cached when lr < mat).
 // cached: every valid row of the wave lies in the cached rows (a choice
 // uniform over the wave, as for CSR rows).
-template <typename V, int FMT, class Op>
+// STREAM: the values are read past the caches' retention (nontemporal).  A large
+// matrix is not in any of them the next iteration, and streaming it leaves the
+// vectors there: 256^3 FP64 494 -> 480 us an iteration, FP32 337 -> 299.
+template <bool STREAM, typename V, int FMT, class Op>
 __device__ __forceinline__ V dia_row(const CgArgs<V>& a, const Lds<V>& c, int i, int lr, bool cached, bool fill,
                                      const Op& op)
 {
@@ -561,7 +611,7 @@ __device__ __forceinline__ V dia_row(const CgArgs<V>& a, const Lds<V>& c, int i,
         const int jc = in ? (int)j : i;
         V mv;
         if (cached && !fill) mv = c.mval[d * c.mat + lr];
-        else mv = a.val[(size_t)d * a.n + i];
+        else mv = STREAM ? __builtin_nontemporal_load(a.val + ((size_t)d * a.n + i)) : a.val[(size_t)d * a.n + i];
         if (cached && fill) c.mval[d * c.mat + lr] = mv;
         const V prod = mv * op(jc);
         s = in ? s + prod : s;
@@ -573,7 +623,8 @@ __device__ __forceinline__ V dia_row(const CgArgs<V>& a, const Lds<V>& c, int i,
 // lane's, and no ballot separates one row's loads from the next row's).
 // MC: the segment may lie in the workgroup's matrix cache (else its entries
 // come straight from HBM, with no per-row choice either).
-template <typename V, int FMT, bool IRR, bool MC, class Op>
+// STREAM: see dia_row.
+template <typename V, int FMT, bool IRR, bool MC, bool STREAM, class Op>
 __device__ __forceinline__ V row_value(const CgArgs<V>& a, const Lds<V>& c, int kb, int i, bool valid, int lr,
                                        bool fill, const Op& op, bool& lng)
 {
@@ -583,12 +634,16 @@ __device__ __forceinline__ V row_value(const CgArgs<V>& a, const Lds<V>& c, int 
         lng = false;
         const int k0 = valid ? a.rowptr[i] : 0;
         const int k1 = valid ? a.rowptr[i + 1] : 0;
-        if constexpr (!MC) return csr_short_from<V>(a.col, a.val, 0, k0, k1, c, kb, false, op);
+        if constexpr (!MC) {
+            if (__ballot((long long)k1 + kCsrChunk > a.nnz) == 0)
+                return csr_short_from<true, V>(a.col, a.val, 0, k0, k1, c, kb, false, op);
+            return csr_short_from<false, V>(a.col, a.val, 0, k0, k1, c, kb, false, op);
+        }
         return csr_short(a, c, kb, k0, k1, __ballot((long long)k1 - kb > (long long)c.mat) == 0, fill, op);
     } else {
         lng = false;
         const bool cached = MC && __ballot(valid && lr >= c.mat) == 0;
-        return valid ? dia_row<V, FMT>(a, c, i, lr, cached, MC && fill, op) : (V)0;
+        return valid ? dia_row<STREAM, V, FMT>(a, c, i, lr, cached, MC && fill, op) : (V)0;
     }
 }
 
@@ -633,7 +688,7 @@ __device__ __forceinline__ V long_value(const CgArgs<V>& a, int j)
 // loads the cached units of x.  Segments holding long rows get their
 // partials in fix_initial.
 template <typename V, int FMT, int NG>
-__device__ void phase_initial(const CgArgs<V>& a, const Lds<V>& c, int me, int kb, bool fill, double* lds)
+__device__ __forceinline__ void phase_initial(const CgArgs<V>& a, const Lds<V>& c, int me, int kb, bool fill, double* lds)
 {
     const int t = lane256();
     const OpVec<V> op{a.x};
@@ -652,7 +707,7 @@ __device__ void phase_initial(const CgArgs<V>& a, const Lds<V>& c, int me, int k
                 bool lng = false;
                 V ax = (V)0;
                 if (!a.x_is_zero)
-                    ax = row_value<V, FMT, decltype(irr)::value, true>(a, c, kb, i, valid, u * kLanes + t, fill, op,
+                    ax = row_value<V, FMT, decltype(irr)::value, true, NG == 1>(a, c, kb, i, valid, u * kLanes + t, fill, op,
                                                                         lng);
                 if (valid) {
                     if (u < c.units[VC_X]) c.vec[VC_X][u * kLanes + t] = a.x[i];
@@ -720,7 +775,7 @@ __device__ __forceinline__ void fix_long_rows(const CgArgs<V>& a, lds_ptr<const 
 }
 
 template <typename V, int FMT, int NG>
-__device__ void fix_initial(const CgArgs<V>& a, const Lds<V>& c, int me, double* lds)
+__device__ __forceinline__ void fix_initial(const CgArgs<V>& a, const Lds<V>& c, int me, double* lds)
 {
     fix_long_rows(
         a, c.slots,
@@ -754,10 +809,13 @@ __device__ void fix_initial(const CgArgs<V>& a, const Lds<V>& c, int me, double*
 }
 
 // Phase 1 of an iteration: p = r + beta*p (stored into pnew), Ap = A p,
-// partials of p.Ap into part_a.
+// partials of p.Ap into part_a.  Also the x update of the iteration before, x =
+// alpha*p + x with that iteration's alpha and p: this phase reads the old p of
+// its rows anyway, so phase 2 need not read p again (one vector of the ten that
+// an iteration moves).  The last one follows the loop.
 template <typename V, int FMT, int NG, bool FIRST>
-__device__ void phase_spmv(const CgArgs<V>& a, const Lds<V>& c, int me, int kb, const V* pold, V* pnew, V beta,
-                           bool fill, double* lds)
+__device__ __forceinline__ void phase_spmv(const CgArgs<V>& a, const Lds<V>& c, int me, int kb, const V* pold, V* pnew, V beta,
+                           V alpha_before, bool fill, double* lds)
 {
     const int t = lane256();
     const OpP<V, FIRST> op{a.r, pold, beta};
@@ -772,17 +830,25 @@ __device__ void phase_spmv(const CgArgs<V>& a, const Lds<V>& c, int me, int kb, 
                 const int i = s * kSeg + kk * kLanes + t;
                 const int u = q * kPerLane + kk;
                 const bool valid = i < a.n;
-                V pi = (V)0;
+                V pi = (V)0, xi = (V)0;
                 if (valid) {
                     const V ri = vget<C>(c, VC_R, u, a.r, i);
-                    pi = FIRST ? ri : ri + beta * vget<C>(c, VC_P, u, pold, i);
+                    if constexpr (FIRST) {
+                        pi = ri;
+                    } else {
+                        const V po = vget<C>(c, VC_P, u, pold, i);
+                        pi = ri + beta * po;
+                        xi = alpha_before * po + vget<C>(c, VC_X, u, a.x, i);
+                    }
                 }
                 bool lng = false;
                 const V api =
-                    row_value<V, FMT, decltype(irr)::value, C>(a, c, kb, i, valid, u * kLanes + t, fill, op, lng);
+                    row_value<V, FMT, decltype(irr)::value, C, NG == 1>(a, c, kb, i, valid, u * kLanes + t, fill, op, lng);
                 if (valid) {
                     vput<C>(c, VC_P, u, pnew, i, pi, true);
                     if (!lng) vput<C>(c, VC_AP, u, a.ap, i, api, false);
+                    // (stored last: the row's loads are not waited for behind it)
+                    if constexpr (!FIRST) vput<C>(c, VC_X, u, a.x, i, xi, false);
                 }
                 sum.add(kk, prod_d(pi, api), valid && !lng);
                 anyl |= lng ? 1 : 0;
@@ -808,7 +874,7 @@ __device__ void phase_spmv(const CgArgs<V>& a, const Lds<V>& c, int me, int kb, 
 }
 
 template <typename V, int FMT, int NG>
-__device__ void fix_spmv(const CgArgs<V>& a, const Lds<V>& c, int me, const V* pnew, double* lds)
+__device__ __forceinline__ void fix_spmv(const CgArgs<V>& a, const Lds<V>& c, int me, const V* pnew, double* lds)
 {
     fix_long_rows(
         a, c.slots,
@@ -830,9 +896,9 @@ __device__ void fix_spmv(const CgArgs<V>& a, const Lds<V>& c, int me, const V* p
         });
 }
 
-// Phase 2: x = alpha*p + x ; r = (-alpha)*Ap + r ; partials of r.r into part_b.
+// Phase 2: r = (-alpha)*Ap + r ; partials of r.r into part_b.
 template <typename V, int FMT, int NG>
-__device__ void phase_update(const CgArgs<V>& a, const Lds<V>& c, int me, const V* pnew, V alpha, double* lds)
+__device__ __forceinline__ void phase_update(const CgArgs<V>& a, const Lds<V>& c, V alpha, double* lds)
 {
     const int t = lane256();
     const V na = -alpha;
@@ -847,9 +913,6 @@ __device__ void phase_update(const CgArgs<V>& a, const Lds<V>& c, int me, const 
                 double v = 0.0;
                 if (i < a.n) {
                     const int u = q * kPerLane + kk;
-                    const V pi = vget<C>(c, VC_P, u, pnew, i);
-                    const V xi = alpha * pi + vget<C>(c, VC_X, u, a.x, i);
-                    vput<C>(c, VC_X, u, a.x, i, xi, false);
                     const V ri = na * vget<C>(c, VC_AP, u, a.ap, i) + vget<C>(c, VC_R, u, a.r, i);
                     vput<C>(c, VC_R, u, a.r, i, ri, true);
                     v = prod_d(ri, ri);
@@ -910,13 +973,14 @@ __global__ void __launch_bounds__(NG * kLanes) cg_persistent_kernel(CgArgs<V> a)
     if (!grid_sync(a.sync, G, a.timeout, false)) return;  // part_a/part_b are rewritten below
 
     double r0 = 0.0;
+    V alpha = (V)0;
     int k = 1;
     V* pold = a.p0;
     V* pnew = a.p1;
     while ((a.static_iter || !(r1 < thr)) && k <= a.max_iter) {
         // ---- p = r + beta*p ; Ap = A p ; partials of p.Ap ----
-        if (k == 1) phase_spmv<V, FMT, NG, true>(a, c, me, kb, pold, pnew, (V)0, fill, lds);
-        else phase_spmv<V, FMT, NG, false>(a, c, me, kb, pold, pnew, (V)(r1 / r0), fill, lds);
+        if (k == 1) phase_spmv<V, FMT, NG, true>(a, c, me, kb, pold, pnew, (V)0, (V)0, fill, lds);
+        else phase_spmv<V, FMT, NG, false>(a, c, me, kb, pold, pnew, (V)(r1 / r0), alpha, fill, lds);
         fill = false;
         if (!grid_sync(a.sync, G, a.timeout, false)) return;
         if (has_long) {
@@ -924,9 +988,9 @@ __global__ void __launch_bounds__(NG * kLanes) cg_persistent_kernel(CgArgs<V> a)
             if (!grid_sync(a.sync, G, a.timeout, false)) return;
         }
         const double pap = reduce_parts<NG>(a.part_a, a.nseg, lds);
-        const double alpha_d = r1 / pap;
-        // ---- x = alpha*p + x ; r = (-alpha)*Ap + r ; partials of r.r ----
-        phase_update<V, FMT, NG>(a, c, me, pnew, (V)alpha_d, lds);
+        alpha = (V)(r1 / pap);
+        // ---- r = (-alpha)*Ap + r ; partials of r.r ----
+        phase_update<V, FMT, NG>(a, c, alpha, lds);
         if (!grid_sync(a.sync, G, a.timeout, false)) return;
         r0 = r1;
         r1 = reduce_parts<NG>(a.part_b, a.nseg, lds);
@@ -936,15 +1000,18 @@ __global__ void __launch_bounds__(NG * kLanes) cg_persistent_kernel(CgArgs<V> a)
         pold = pnew;
         pnew = tmp;
     }
-    // ---- the cached units of x go back to HBM ----
-    if (c.units[VC_X] > 0) {
+    // ---- the last x update; the cached units of x go back to HBM ----
+    if (k > 1 || c.units[VC_X] > 0) {
         const int l = lane256();
         for_owned(a, c.slots, [&](int s, int q) {
-            for (int k = 0; k < kPerThread<NG>; ++k) {
-                const int kk = first_row<NG>() + k;
+            for (int j = 0; j < kPerThread<NG>; ++j) {
+                const int kk = first_row<NG>() + j;
                 const int u = q * kPerLane + kk;
                 const int i = s * kSeg + kk * kLanes + l;
-                if (u < c.units[VC_X] && i < a.n) a.x[i] = c.vec[VC_X][u * kLanes + l];
+                if (i >= a.n) continue;
+                V xi = vget(c, VC_X, u, a.x, i);
+                if (k > 1) xi = alpha * vget(c, VC_P, u, pold, i) + xi;
+                a.x[i] = xi;
             }
         });
     }
@@ -1328,6 +1395,7 @@ int cg_solve(int fmt, const perks_csr* csr, const perks_dia* dia, const double* 
             a.rowptr = csr->rowptr;
             a.col = csr->col;
             a.val = csr->val;
+            a.nnz = csr->nnz;
         } else {
             a.val = dia->val;
             a.ndiag = dia->ndiag;
@@ -1442,6 +1510,7 @@ int cg_solve(int fmt, const perks_csr* csr, const perks_dia* dia, const double* 
             if (fmt == FMT_CSR) {
                 f.rowptr = csr->rowptr;
                 f.col = csr->col;
+                f.nnz = csr->nnz;
             } else {
                 f.ndiag = dia->ndiag;
                 for (int d = 0; d < dia->ndiag; ++d) f.offs[d] = dia->offsets[d];
@@ -1535,6 +1604,7 @@ int cg_solve_f32(int fmt, const perks_csr_f32* csr, const perks_dia_f32* dia, co
         f.rowptr = csr->rowptr;
         f.col = csr->col;
         f.val = csr->val;
+        f.nnz = csr->nnz;
     } else {
         f.ndiag = dia->ndiag;
         for (int d = 0; d < dia->ndiag; ++d) f.offs[d] = dia->offsets[d];
