@@ -8,8 +8,10 @@
 //
 // Two kernels serve these shapes: the register-streaming kernel
 // (j3d_stream_kernel.h; one wave per 64 x 8 tile, planes in VGPRs; the
-// default, 1.6-3.7x the other per step at 512^3) and the LDS-plane kernel
-// (j3d_general_kernel.h; a workgroup per 64 x 16/32 tile, planes in LDS).
+// default, 1.6-3.7x the other per step at 512^3; the 17- and 27-point shapes run
+// its plane-by-plane form, j3d_sweep_kernel.h, up to the sizes of sweep_limit)
+// and the LDS-plane kernel (j3d_general_kernel.h; a workgroup per 64 x 16/32
+// tile, planes in LDS).
 // opts->tune[4] picks one: 2 = streaming, 3 = LDS planes, 0 = default.
 #include "j3d_general.h"
 
@@ -19,6 +21,7 @@
 #include "api_common.h"
 #include "j3d_general_kernel.h"
 #include "j3d_stream_kernel.h"
+#include "j3d_sweep_kernel.h"
 
 namespace perks {
 
@@ -42,6 +45,17 @@ void* stream_kernel_for(int dtype, int shape, int bc, int rows)
     case PERKS_F32: return j3s_kernel_f32(shape, bc, rows);
     case PERKS_F16: return j3s_kernel_f16(shape, bc, rows);
     case PERKS_BF16: return j3s_kernel_bf16(shape, bc, rows);
+    default: return nullptr;
+    }
+}
+
+void* sweep_kernel_for(int dtype, int shape, int bc, bool has_div)
+{
+    switch (dtype) {
+    case PERKS_F64: return j3z_kernel_f64(shape, bc, has_div);
+    case PERKS_F32: return j3z_kernel_f32(shape, bc, has_div);
+    case PERKS_F16: return j3z_kernel_f16(shape, bc, has_div);
+    case PERKS_BF16: return j3z_kernel_bf16(shape, bc, has_div);
     default: return nullptr;
     }
 }
@@ -71,6 +85,47 @@ int stream_rows(int dtype, int radius, const perks_stencil_opts* o)
     if (o->tune[4] == 4) return j3s::kRowsTall;
     if (o->tune[4] == 2) return j3s::kRows;
     return default_stream_rows(dtype, radius, o->method);
+}
+
+int elem_size(int dtype) { return dtype == PERKS_F64 ? 8 : (dtype == PERKS_F32 ? 4 : 2); }
+
+// The largest pair of fields (bytes) the plane-by-plane form is taken for.  It
+// halves the arithmetic of a stored cell, so it wins wherever the vector units
+// bound the windowed kernel: all 16-bit storage, all FP32 27-point.  Where
+// memory does, the windowed kernel moves less: two steps per pass (persistent),
+// taller tiles (plain).  ms for 50 steps, windowed -> plane by plane:
+//   FP64 17 points  persistent 256^3 3.53 -> 2.16, 288^3 4.46 -> 4.64, 352^3 7.7 -> 8.8, 512^3 21.4 -> 30.4
+//                   plain      256^3 4.35 -> 2.19, 352^3 8.34 -> 7.66, 384^3 10.8 -> 11.1, 512^3 23.9 -> 25.4
+//   FP64 27 points  persistent 256^3 4.64 -> 2.70, 448^3 20.8 -> 16.5, 512^3 28.2 -> 31.2
+//   FP32 17 points  plain      448^3 10.2 -> 9.4, 512^3 15.1 -> 15.5, 640^3 28.0 -> 29.3
+size_t sweep_limit(int dtype, int shape, int method)
+{
+    const bool plain = method == PERKS_METHOD_PLAIN;
+    const size_t MB = 1u << 20;
+    if (elem_size(dtype) == 2) return SIZE_MAX;
+    if (shape == PERKS_SHAPE_3D_TYPE0_R1 && plain) return 768 * MB;
+    if (dtype == PERKS_F64 && !plain) return shape == PERKS_SHAPE_3D_TYPE0_R1 ? 320 * MB : 1536 * MB;
+    return SIZE_MAX;
+}
+
+// The plane-by-plane form runs the shapes whose table allows it, at one step per
+// pass, in place of the short tile.  A persistent grid held to one workgroup per
+// CU keeps the two-step kernel, and with it the plan reported for that limit.
+bool use_sweep(int dtype, int shape, const perks_stencil_opts* o, int levels, size_t cells)
+{
+    if (o->method != PERKS_METHOD_PLAIN && (o->blkpsm == 1 || o->tune[3] == 1)) return false;
+    return levels == 1 && (o->tune[4] == 0 || o->tune[4] == 2) && j3z::sweeps(shape) &&
+           2 * cells * elem_size(dtype) <= sweep_limit(dtype, shape, o->method);
+}
+
+// Cells a tile of the register-streaming kernels stores, and the ghost planes of a slab.
+struct TileGeom {
+    int vw, vh, ghost;
+};
+TileGeom stream_geom(bool sweep, int radius, int levels, int rows)
+{
+    if (sweep) return {j3z::kSweepCols, j3z::kSweepRows, 2};
+    return {64 - 2 * radius * levels, rows - 2 * radius * levels, 2 * radius * levels};
 }
 
 constexpr int kStreamItems = 16384;  // per-step launches: work items (waves) to aim for
@@ -112,16 +167,45 @@ int best_slabs(int nz, long long tiles_xy, int G, int ghost)
     return best;
 }
 
+// The same for the plane-by-plane form: a pass takes the stages of an item times
+// the items of the SIMD that gets most.  A wave alone on its SIMD issues FP64
+// cells as fast as two do, and other formats' (whose loads return less per
+// request) some 1.2 times slower.  With `waves` resident ones (persistent; 0:
+// items start as others end) none gets a second item while the first can be made
+// longer instead (352^3 FP64 27 points: 15 slabs in two rounds 11.0 ms, 7 in one
+// 8.6), and the barrier costs some 3 stages for every wave of a SIMD (128^3 FP64
+// 27 points: three waves per SIMD 0.98 ms, one 0.77; 320^3: two 6.35, one 5.65).
+int sweep_slabs(int dtype, int nz, long long tiles_xy, int cus, long long waves)
+{
+    const long long simds = 4LL * cus;
+    const double lone = dtype != PERKS_F64 ? 1.2 : (waves > 0 ? 1.0 : 1.05);
+    int best = 1;
+    double best_cost = 1e300;
+    const int cap = std::min(nz, 512);
+    for (int s = 1; s <= cap; ++s) {
+        const long long items = tiles_xy * s;
+        if (waves > 0 && s > 1 && items > waves) break;
+        const double share = (double)((items + simds - 1) / simds);
+        const double cost = std::max(lone, share) * j3z::sweep_stages((nz + s - 1) / s) + (waves > 0 ? 3 * share : 0);
+        if (cost < best_cost * 0.999) {
+            best_cost = cost;
+            best = s;
+        }
+    }
+    return best;
+}
+
 }  // namespace
 
-int j3g_levels(int dtype, int shape, const perks_stencil_opts* o)
+int j3g_levels(int dtype, int shape, const perks_stencil_opts* o, size_t cells)
 {
     const ShapeDesc* sd = shape_by_id(shape);
     if (!sd) return 1;
     if (o->method == PERKS_METHOD_PLAIN) return 1;
     if (use_stream(o, sd->radius)) {
         const int lm = j3s::stream3_max_levels(sd->radius);
-        return o->tune[2] > 0 ? std::min(o->tune[2], lm) : lm;
+        if (o->tune[2] <= 0) return use_sweep(dtype, shape, o, 1, cells) ? 1 : lm;
+        return std::min(o->tune[2], lm);
     }
     int tx, ty;
     tile_of(dtype, &tx, &ty);
@@ -132,19 +216,24 @@ int j3g_levels(int dtype, int shape, const perks_stencil_opts* o)
     return std::max(1, std::min(L, maxL));
 }
 
-int j3g_plan(int dtype, int nz, int ny, int nx, const perks_stencil_opts* o, const perks_device_caps* caps,
+int j3g_plan(int dtype, int nz, int ny, int nx, const perks_stencil_opts* opts, const perks_device_caps* caps,
              int occupancy, perks_plan_info* out)
 {
-    const ShapeDesc* sd = shape_by_id(o->shape);
+    const ShapeDesc* sd = shape_by_id(opts->shape);
     if (!sd || sd->dims != 3 || !caps || !out) return PERKS_ERR_INVALID_ARG;
+    perks_stencil_opts lim = *opts;
+    if (occupancy == 1) lim.blkpsm = 1;
+    const perks_stencil_opts* o = &lim;
     int tx, ty;
     tile_of(dtype, &tx, &ty);
     const int R = sd->radius;
-    const int L = j3g_levels(dtype, o->shape, o);
+    const size_t cells = (size_t)nz * ny * nx;
+    const int L = j3g_levels(dtype, o->shape, o, cells);
     if (use_stream(o, R)) {
         const int rows = stream_rows(dtype, R, o);
-        const int VW = 64 - 2 * R * L, VH = rows - 2 * R * L;
-        const long long tiles_xy = (long long)((nx + VW - 1) / VW) * ((ny + VH - 1) / VH);
+        const bool sweep = use_sweep(dtype, o->shape, o, L, cells);
+        const TileGeom tg = stream_geom(sweep, R, L, rows);
+        const long long tiles_xy = (long long)((nx + tg.vw - 1) / tg.vw) * ((ny + tg.vh - 1) / tg.vh);
         std::memset(out, 0, sizeof(*out));
         out->block = j3s::kWaves * 64;
         out->tile_x = 64;
@@ -153,7 +242,9 @@ int j3g_plan(int dtype, int nz, int ny, int nx, const perks_stencil_opts* o, con
         int nzs = 1;
         long long groups = 0;
         if (o->method == PERKS_METHOD_PLAIN) {
-            nzs = (int)std::max(1LL, std::min<long long>(nz, (kStreamItems + tiles_xy - 1) / tiles_xy));
+            nzs = sweep
+                      ? sweep_slabs(dtype, nz, tiles_xy, caps->cu_count, 0)
+                      : (int)std::max(1LL, std::min<long long>(nz, (kStreamItems + tiles_xy - 1) / tiles_xy));
             groups = (tiles_xy * nzs + j3s::kWaves - 1) / j3s::kWaves;
         } else {
             if (occupancy <= 0) return PERKS_ERR_NOT_LAUNCHABLE;
@@ -161,7 +252,8 @@ int j3g_plan(int dtype, int nz, int ny, int nx, const perks_stencil_opts* o, con
             if (o->blkpsm > 0 && o->blkpsm < occ) occ = o->blkpsm;
             if (o->tune[3] > 0 && o->tune[3] < occ) occ = o->tune[3];
             const int G = caps->cu_count * occ;
-            nzs = best_slabs(nz, tiles_xy, G * j3s::kWaves, 2 * R * L);
+            nzs = sweep ? sweep_slabs(dtype, nz, tiles_xy, caps->cu_count, (long long)G * j3s::kWaves)
+                        : best_slabs(nz, tiles_xy, G * j3s::kWaves, tg.ghost);
             groups = std::min<long long>(G, (tiles_xy * nzs + j3s::kWaves - 1) / j3s::kWaves);
             out->occupancy = occ;
         }
@@ -198,15 +290,17 @@ int j3g_plan(int dtype, int nz, int ny, int nx, const perks_stencil_opts* o, con
     return PERKS_OK;
 }
 
-void* j3g_fn(int dtype, const perks_stencil_opts* o, int* block, size_t* lds)
+void* j3g_fn(int dtype, const perks_stencil_opts* o, size_t cells, int* block, size_t* lds)
 {
     const ShapeDesc* sd = shape_by_id(o->shape);
     if (!sd || sd->dims != 3) return nullptr;
     const bool streaming = use_stream(o, sd->radius);
     if (block) *block = streaming ? j3s::kWaves * 64 : j3g::kThreads;
-    if (lds) *lds = streaming ? 0 : lds_for(dtype, sd->radius, j3g_levels(dtype, o->shape, o));
-    return streaming ? stream_kernel_for(dtype, o->shape, o->boundary, stream_rows(dtype, sd->radius, o))
-                     : kernel_for(dtype, o->shape, o->boundary);
+    if (lds) *lds = streaming ? 0 : lds_for(dtype, sd->radius, j3g_levels(dtype, o->shape, o, cells));
+    if (!streaming) return kernel_for(dtype, o->shape, o->boundary);
+    if (use_sweep(dtype, o->shape, o, j3g_levels(dtype, o->shape, o, cells), cells))
+        return sweep_kernel_for(dtype, o->shape, o->boundary, o->use_ref_coefs ? sd->divisor != 0.0 : o->divisor != 0.0);
+    return stream_kernel_for(dtype, o->shape, o->boundary, stream_rows(dtype, sd->radius, o));
 }
 
 int j3g_run(int dtype, void* d_a, void* d_b, int nz, int ny, int nx, int steps, const KCoefs& cf,
@@ -217,7 +311,12 @@ int j3g_run(int dtype, void* d_a, void* d_b, int nz, int ny, int nx, int steps, 
     const int R = sd->radius;
     const bool streaming = use_stream(o, R);
     const int rows = streaming ? stream_rows(dtype, R, o) : 0;
-    void* fn = streaming ? stream_kernel_for(dtype, o->shape, o->boundary, rows) : kernel_for(dtype, o->shape, o->boundary);
+    const size_t cells = (size_t)nz * ny * nx;
+    const int L = j3g_levels(dtype, o->shape, o, cells);
+    const bool sweep = streaming && use_sweep(dtype, o->shape, o, L, cells);
+    void* fn = sweep ? sweep_kernel_for(dtype, o->shape, o->boundary, cf.divisor != 0.0)
+                     : (streaming ? stream_kernel_for(dtype, o->shape, o->boundary, rows)
+                                  : kernel_for(dtype, o->shape, o->boundary));
     if (!fn) return PERKS_ERR_UNSUPPORTED;
     perks_device_caps caps;
     int rc = device_caps_cached(&caps);
@@ -228,12 +327,12 @@ int j3g_run(int dtype, void* d_a, void* d_b, int nz, int ny, int nx, int steps, 
         tx = 64;
         ty = rows;
     }
-    const int L = j3g_levels(dtype, o->shape, o);
     const size_t lds = streaming ? 0 : lds_for(dtype, R, L);
     const int threads = streaming ? j3s::kWaves * 64 : j3g::kThreads;
     const int per_group = streaming ? j3s::kWaves : 1;  // work items per workgroup
-    const int VW = tx - 2 * R * L, VH = ty - 2 * R * L;
-    const long long tiles_xy = (long long)((nx + VW - 1) / VW) * ((ny + VH - 1) / VH);
+    const TileGeom tg = streaming ? stream_geom(sweep, R, L, rows)
+                                  : TileGeom{tx - 2 * R * L, ty - 2 * R * L, 2 * R * L};
+    const long long tiles_xy = (long long)((nx + tg.vw - 1) / tg.vw) * ((ny + tg.vh - 1) / tg.vh);
 
     j3g::J3gArgs a;
     std::memset(&a, 0, sizeof(a));
@@ -266,7 +365,8 @@ int j3g_run(int dtype, void* d_a, void* d_b, int nz, int ny, int nx, int steps, 
         // workgroup, enough slabs for about eight workgroups per CU; streaming
         // kernel: one item per wave, enough slabs for kStreamItems items.
         const long long want = streaming ? kStreamItems : 8LL * caps.cu_count;
-        a.nzs = (int)std::max(1LL, std::min<long long>(nz, (want + tiles_xy - 1) / tiles_xy));
+        a.nzs = sweep ? sweep_slabs(dtype, nz, tiles_xy, caps.cu_count, 0)
+                      : (int)std::max(1LL, std::min<long long>(nz, (want + tiles_xy - 1) / tiles_xy));
         const long long nitems = tiles_xy * a.nzs;
         if (nitems > 0x7fffffffLL) return PERKS_ERR_UNSUPPORTED_SIZE;
         grid = (int)((nitems + per_group - 1) / per_group);
@@ -283,7 +383,8 @@ int j3g_run(int dtype, void* d_a, void* d_b, int nz, int ny, int nx, int steps, 
         if (o->blkpsm > 0 && o->blkpsm < occ) occ = o->blkpsm;
         if (o->tune[3] > 0 && o->tune[3] < occ) occ = o->tune[3];
         const int G = caps.cu_count * occ;
-        a.nzs = best_slabs(nz, tiles_xy, G * per_group, 2 * R * L);
+        a.nzs = sweep ? sweep_slabs(dtype, nz, tiles_xy, caps.cu_count, (long long)G * per_group)
+                      : best_slabs(nz, tiles_xy, G * per_group, tg.ghost);
         grid = (int)std::min<long long>(G, (tiles_xy * a.nzs + per_group - 1) / per_group);
         a.npass = npass;
         a.step_offset = 0;

@@ -31,6 +31,7 @@ namespace perks {
 namespace {
 
 constexpr int kDefaultSampleSteps = 12;  // a multiple of every pass depth (1..4)
+constexpr int kMaxLevels = 4;            // pass depths tried
 
 struct Candidate {
     int method;
@@ -60,15 +61,16 @@ std::vector<Candidate> candidates(int dtype, const perks_stencil_opts* o)
         c.push_back({PERKS_METHOD_PLAIN, 0, 1});
         const int nv = j3d_persistent_variants();
         for (int v = 0; v < nv; ++v) {
-            for (int l = 1; l <= 4; ++l) c.push_back({PERKS_METHOD_PERSISTENT, v, l});
+            for (int l = 1; l <= kMaxLevels; ++l) c.push_back({PERKS_METHOD_PERSISTENT, v, l});
         }
         c.push_back({PERKS_METHOD_PERSISTENT, kResidentVariant, 1});  // resident tiles: one step per barrier
         return c;
     }
     for (int k : {2, 4, 3}) {  // register streaming (short and tall tiles), LDS planes
         c.push_back({PERKS_METHOD_PLAIN, k, 1});
-        perks_stencil_opts p = with(o, {PERKS_METHOD_PERSISTENT, k, 0});
-        const int maxl = j3g_levels(dtype, o->shape, &p);
+        // the most levels, not the default for a size
+        perks_stencil_opts p = with(o, {PERKS_METHOD_PERSISTENT, k, kMaxLevels});
+        const int maxl = j3g_levels(dtype, o->shape, &p, 0);
         for (int l = 1; l <= maxl; ++l) c.push_back({PERKS_METHOD_PERSISTENT, k, l});
     }
     return c;
@@ -102,7 +104,7 @@ int describe(int dtype, int nz, int ny, int nx, const perks_stencil_opts* base, 
                                    &block);
         }
     } else {
-        fn = j3g_fn(dtype, &o, &block, &lds);
+        fn = j3g_fn(dtype, &o, (size_t)nz * ny * nx, &block, &lds);
     }
     out->block = block;
     if (!fn) return out->status = PERKS_ERR_UNSUPPORTED;
