@@ -37,6 +37,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 
@@ -103,28 +104,117 @@ int tile_width(const Variant& v, int l) { return v.pair ? 128 - 4 * ((l + 1) / 2
 // Makespan model of one pass with `l` levels: items are dealt round-robin to
 // G workgroups; an item costs its slab height plus the 2*l ghost planes it
 // reads beyond the slab.  Picks the z-slab count that minimises
-// rounds * (planes per item).
-static int best_nzs(int nz, int ny, int ntx, int l, int G, int rows)
+// rounds * (planes per item).  `planes`: what a workgroup marches then, less
+// the ghost planes the slabs at the domain's ends do not have.
+static int best_nzs(int nz, int ny, int ntx, int l, int G, int rows, double* planes)
 {
     const long long tiles = (long long)ntx * j3dp::y_tiles(ny, rows, l);
     int best = 1;
-    double best_cost = 1e300;
+    double best_cost = 1e300, best_rounds = 0;
     const int cap = nz < 256 ? nz : 256;
     for (int s = 1; s <= cap; ++s) {
         const long long items = tiles * s;
         const long long rounds = (items + G - 1) / G;
+        if ((double)rounds * 2.0 * l >= best_cost) break;  // rounds only grow from here
         const double per = (double)(nz + s - 1) / s + 2.0 * l;
         const double cost = (double)rounds * per;
         if (cost < best_cost - 1e-9) {
             best_cost = cost;
+            best_rounds = (double)rounds;
             best = s;
         }
     }
+    *planes = best_cost - 0.384 * l * best_rounds;
     return best;
 }
 
-int plan_persistent(int dtype, int nz, int ny, int nx, const perks_stencil_opts* o, const perks_device_caps* caps,
-                    int occupancy, perks_plan_info* out)
+// Slabs per level count of a variant: nzs[l], and the planes a workgroup
+// marches per pass.
+struct Split {
+    int nzs[kMaxLevels + 1];
+    double planes[kMaxLevels + 1];
+};
+static Split split_domain(const Variant& v, int nz, int ny, int nx, int bc, int G)
+{
+    Split s;
+    for (int l = 1; l <= kMaxLevels; ++l) {
+        // x tiles as the kernel cuts them (j3dp::x_tiles; the two-column form
+        // keeps ghost lanes at both faces)
+        const int ntx = v.pair ? (nx + tile_width(v, l) - 1) / tile_width(v, l) : j3dp::x_tiles(bc, nx, l);
+        s.nzs[l] = best_nzs(nz, ny, ntx, l, G, v.nw * v.ny, &s.planes[l]);
+    }
+    return s;
+}
+
+// Microseconds of one pass of `l` levels: a barrier and a fill, and planes at a
+// rate per level of the format's update (with the boundary step of tiles that
+// have ghost lanes beyond an x face: always under clamp, on narrow grids under
+// zero) -- and, where the fields exceed the last-level cache, the traffic with
+// it.  Fitted to passes of 2, 3 and 4 levels over 26 domains from 32^3 to 512^3,
+// odd and flat ones among them, in five formats and both boundaries.
+static double pass_us(int dtype, bool sr, int bc, int nx, double cells, double planes, int l, double width)
+{
+    const bool clamp = bc == PERKS_BC_CLAMP;
+    double a;
+    switch (dtype) {
+    case PERKS_F32: a = clamp ? 0.502 : 0.296; break;
+    case PERKS_F64: a = clamp ? 0.548 : 0.321; break;
+    default: a = sr ? (clamp ? 0.75 : 0.52) : (clamp ? 0.549 : 0.321); break;
+    }
+    if (!clamp && !j3dp::x_face_tiles(bc, nx, l)) a *= 1.266;
+    double t = 6.87 + planes * width * a * (l + (clamp ? 0.073 : 0.41));
+    const double bytes = 2.0 * cells * elem_bytes(dtype);
+    if (bytes > 270e6) t = std::sqrt(t * t + bytes / 4.43e6 * (bytes / 4.43e6));
+    return t;
+}
+// ... and of `steps` steps in passes of up to L (0: of many, per step).
+static double run_us(int dtype, bool sr, int bc, int nx, double cells, const Split& s, int steps, int L,
+                     double width)
+{
+    const double full = pass_us(dtype, sr, bc, nx, cells, s.planes[L], L, width);
+    if (steps <= 0) return full / L;
+    const int rest = steps % L;
+    return steps / L * full + (rest ? pass_us(dtype, sr, bc, nx, cells, s.planes[rest], rest, width) : 0.0);
+}
+
+// Where the caller leaves variant, levels and slabs open, the pass is not always
+// the one that is best at 512^3.  A domain that leaves each workgroup a few
+// planes beside the 2L it reads beyond them is faster with fewer levels; in FP32
+// arithmetic a plane of the 16 x 2-row workgroup takes 0.59 of the 16 x 4 one's
+// time, which pays until the chip is full; and tile and round counts jump with
+// the sides.  The default stays unless the model finds 4% in a change.  Over
+// the combinations above at 24, 20 and 10 steps: 9% less time (geometric mean),
+// none more than 2% slower.  us for 24 steps, 4 levels (16-bit clamp: 3) of variant 0 -> chosen:
+//   FP64 zero 64^3 130 -> 109 (3 levels), 256^3 618 -> 553 (3), 260 x 61 x 700 645 -> 381 (3)
+//   FP32 clamp 64^3 137 -> 102, 128^3 190 -> 156 (variant 3, 4 levels), 150 x 250 x 350 429 -> 340 (2 levels)
+//   BF16 stochastic 128^3 219 -> 177 (variant 3)
+constexpr int kShortVariant = 3;
+constexpr double kShortWidth = 0.589;
+static_assert(j3dp::kVarF32[0].nw == j3dp::kVarF32[kShortVariant].nw, "the two share a workgroup size and occupancy");
+
+static void choose(int dtype, bool sr, int bc, int nz, int ny, int nx, int G, int steps, int* var, int* L, Split* s)
+{
+    const double cells = (double)nz * ny * nx;
+    double best = 0.96 * run_us(dtype, sr, bc, nx, cells, *s, steps, *L, 1.0);
+    const Split own = *s;
+    const bool shorter = dtype != PERKS_F64;
+    const Split other = shorter ? split_domain(variant_shape(dtype, kShortVariant), nz, ny, nx, bc, G) : own;
+    for (int v = 0; v <= (shorter ? 1 : 0); ++v) {
+        for (int l = 2; l <= kMaxLevels; ++l) {
+            const double t = run_us(dtype, sr, bc, nx, cells, v ? other : own, steps, l, v ? kShortWidth : 1.0);
+            if (t < best) {
+                best = t;
+                *var = v ? kShortVariant : 0;
+                *L = l;
+                *s = v ? other : own;
+            }
+        }
+    }
+}
+
+// The plan of `steps` steps (0: many) and the variant it runs.
+static int plan_steps(int dtype, int nz, int ny, int nx, int steps, const perks_stencil_opts* o,
+                      const perks_device_caps* caps, int occupancy, int* var, perks_plan_info* out)
 {
     if (o->shape != PERKS_SHAPE_3D_STAR_R1) return PERKS_ERR_UNSUPPORTED;
     if ((long long)ny * nx * elem_bytes(dtype) >= (long long)kOob) return PERKS_ERR_UNSUPPORTED_SIZE;
@@ -134,16 +224,22 @@ int plan_persistent(int dtype, int nz, int ny, int nx, const perks_stencil_opts*
         if (o->blkpsm > 0 && o->blkpsm < occ) occ = o->blkpsm;
         return plan_resident(dtype, nz, ny, nx, caps, occ, out);
     }
-    const Variant v = variant_shape(dtype, variant_of(o));
+    *var = variant_of(o);
+    Variant v = variant_shape(dtype, *var);
     if (v.pair && (nx & 1)) return PERKS_ERR_UNSUPPORTED;  // two columns per lane need an even width
     int occ = std::min(occupancy, std::max(1, kCoopMaxWavesPerCu / v.nw));
     if (o->blkpsm > 0 && o->blkpsm < occ) occ = o->blkpsm;
     if (o->tune[3] > 0 && o->tune[3] < occ) occ = o->tune[3];
     const int G = caps->cu_count * occ;
     if (G <= 0) return PERKS_ERR_NOT_LAUNCHABLE;
-    int L = o->tune[2] > 0 ? o->tune[2]
-                           : default_levels(dtype, o->rounding == PERKS_ROUND_STOCHASTIC, o->boundary, nx);
+    const bool sr = o->rounding == PERKS_ROUND_STOCHASTIC;
+    int L = o->tune[2] > 0 ? o->tune[2] : default_levels(dtype, sr, o->boundary, nx);
     if (L > kMaxLevels) L = kMaxLevels;
+    Split split = split_domain(v, nz, ny, nx, o->boundary, G);
+    if (o->tune[2] <= 0 && o->tune[4] == 0 && o->tune[7] <= 0) {
+        choose(dtype, sr, o->boundary, nz, ny, nx, G, steps, var, &L, &split);
+        v = variant_shape(dtype, *var);
+    }
     std::memset(out, 0, sizeof(*out));
     out->grid[0] = G;
     out->grid[1] = 1;
@@ -154,14 +250,15 @@ int plan_persistent(int dtype, int nz, int ny, int nx, const perks_stencil_opts*
     out->tile_x = v.pair ? 128 : 64;
     out->tile_y = v.nw * v.ny;
     out->reserved[0] = L;
-    for (int l = 1; l <= kMaxLevels; ++l)
-    {
-        // x tiles as the kernel cuts them (j3dp::x_tiles; the two-column form
-        // keeps ghost lanes at both faces)
-        const int ntx = v.pair ? (nx + tile_width(v, l) - 1) / tile_width(v, l) : j3dp::x_tiles(o->boundary, nx, l);
-        out->reserved[l] = o->tune[7] > 0 ? std::min(o->tune[7], nz) : best_nzs(nz, ny, ntx, l, G, v.nw * v.ny);
-    }
+    for (int l = 1; l <= kMaxLevels; ++l) out->reserved[l] = o->tune[7] > 0 ? std::min(o->tune[7], nz) : split.nzs[l];
     return PERKS_OK;
+}
+
+int plan_persistent(int dtype, int nz, int ny, int nx, const perks_stencil_opts* o, const perks_device_caps* caps,
+                    int occupancy, perks_plan_info* out)
+{
+    int var;
+    return plan_steps(dtype, nz, ny, nx, 0, o, caps, occupancy, &var, out);
 }
 
 // The reference's getminHeight (j3d.cu:598,612) is the domain height at which
@@ -253,18 +350,21 @@ int run_persistent_fmt(int dtype, void* d_a, void* d_b, int nz, int ny, int nx, 
     if (rc != PERKS_OK) return rc;
     if (!caps.cooperative) return PERKS_ERR_NOT_LAUNCHABLE;
     const bool has_div = cf.divisor != 0.0;
-    const int var = variant_of(o);
+    const bool sr = o->rounding == PERKS_ROUND_STOCHASTIC;
     // tune[6] = 1: the contracted update (FP64/FP32 without a divisor; the
     // kernel pickers return nullptr for the rest)
-    void* fn = pick_kernel(dtype, o->boundary, has_div, var, o->rounding == PERKS_ROUND_STOCHASTIC,
-                           j3d_persistent_update(dtype, o, cf));
+    const int up = j3d_persistent_update(dtype, o, cf);
+    int var = variant_of(o);
+    void* fn = pick_kernel(dtype, o->boundary, has_div, var, sr, up);
     if (!fn) return PERKS_ERR_UNSUPPORTED;
     int occ = 0;
     PERKS_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void*>(fn),
                                                                variant_shape(dtype, var).nw * 64, 0));
     perks_plan_info pl;
-    rc = plan_persistent(dtype, nz, ny, nx, o, &caps, occ, &pl);
+    rc = plan_steps(dtype, nz, ny, nx, steps, o, &caps, occ, &var, &pl);
     if (rc != PERKS_OK) return rc;
+    fn = pick_kernel(dtype, o->boundary, has_div, var, sr, up);
+    if (!fn) return PERKS_ERR_UNSUPPORTED;
 
     SyncLease lease;
     rc = lease.acquire();
