@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "api_common.h"
+#include "host_copy.h"
 #include "j2d.h"
 
 namespace perks {
@@ -66,11 +67,12 @@ int host2(int dtype, const T* h_in, int wy, int wx, T* h_out, int steps, const p
             rc = device2(dtype, d_a, d_b, wy, wx, ws, o, nullptr, r);
             if (rc != PERKS_OK) break;
         }
-        if (hipMemcpy(d_a, h_in, bytes, hipMemcpyHostToDevice) != hipSuccess) { rc = PERKS_ERR_HIP; break; }
+        rc = copy_to_device(d_a, h_in, bytes);
+        if (rc != PERKS_OK) break;
         rc = device2(dtype, d_a, d_b, wy, wx, steps, o, nullptr, r);
         if (rc != PERKS_OK) break;
         const T* res = r->result_in_b ? d_b : d_a;
-        if (hipMemcpy(h_out, res, bytes, hipMemcpyDeviceToHost) != hipSuccess) { rc = PERKS_ERR_HIP; break; }
+        rc = copy_to_host(h_out, res, bytes);
     } while (0);
     (void)hipFree(d_a);
     (void)hipFree(d_b);

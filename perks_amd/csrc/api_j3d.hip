@@ -13,6 +13,7 @@
 #include <mutex>
 
 #include "api_common.h"
+#include "host_copy.h"
 #include "j3d_kernels.h"
 #include "storage16.h"
 #include "j3d_general.h"
@@ -223,11 +224,12 @@ int j3d_host(const T* h_in, int nz, int ny, int nx, T* h_out, int steps, const p
             rc = j3d_device<T>(d_a, d_b, nz, ny, nx, ws, o, nullptr, r);
             if (rc != PERKS_OK) break;
         }
-        if (hipMemcpy(d_a, h_in, bytes, hipMemcpyHostToDevice) != hipSuccess) { rc = PERKS_ERR_HIP; break; }
+        rc = copy_to_device(d_a, h_in, bytes);
+        if (rc != PERKS_OK) break;
         rc = j3d_device<T>(d_a, d_b, nz, ny, nx, steps, o, nullptr, r);
         if (rc != PERKS_OK) break;
         const T* res = r->result_in_b ? d_b : d_a;
-        if (hipMemcpy(h_out, res, bytes, hipMemcpyDeviceToHost) != hipSuccess) { rc = PERKS_ERR_HIP; break; }
+        rc = copy_to_host(h_out, res, bytes);
     } while (0);
     (void)hipFree(d_a);
     (void)hipFree(d_b);

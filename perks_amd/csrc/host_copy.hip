@@ -1,0 +1,232 @@
+// host_copy.hip -- copies between pageable host memory and the device, through
+// pinned buffers that several threads fill or empty.
+//
+// What bounds a pageable copy is the host's side of it: the link moves 64 MiB in
+// 1.18 ms either way, one thread's memcpy takes 2.1 ms, four threads' 0.9 ms, and
+// hipMemcpy on pageable memory 2.25 ms to the device and 3.9 ms back (256^3 FP32).
+// Here a copy is cut into pieces that threads take in turn, each through one of
+// kBuffers pinned buffers: while some are copied by the host, others are on the
+// link.  The threads live for one copy (some 20 us each to start).  A host call of
+// 10 steps at 256^3 FP32: 6.8 -> 4.0 ms.
+#include "host_copy.h"
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <exception>
+#include <mutex>
+#include <new>
+#include <thread>
+#include <vector>
+
+#include "api_common.h"
+
+namespace perks {
+
+namespace {
+
+// 17 us of the link go by between two pieces: 64 MiB in pieces of 1, 2 and 4 MiB
+// take 2.16, 1.73 and 1.55 ms; 8 buffers or threads, the same.
+constexpr size_t kPiece = (size_t)4 << 20;
+constexpr int kBuffers = 4;
+constexpr int kThreads = 4;                // with the caller's
+constexpr size_t kMinStaged = 2 * kPiece;  // below, there is nothing to overlap
+constexpr int kMaxIdle = 2;                // sets kept between calls (16 MiB each); more are freed on return
+
+// Pinned buffers of one copy, and an event per buffer.
+struct Staging {
+    int dev = -1;
+    char* mem = nullptr;
+    hipEvent_t ev[kBuffers] = {};
+
+    bool create()
+    {
+        if (hipGetDevice(&dev) != hipSuccess) return false;
+        if (hipHostMalloc((void**)&mem, kPiece * kBuffers, hipHostMallocDefault) != hipSuccess) {
+            mem = nullptr;
+            return false;
+        }
+        for (hipEvent_t& e : ev) {
+            if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+                e = nullptr;
+                return false;
+            }
+        }
+        return true;
+    }
+    void destroy()
+    {
+        for (hipEvent_t e : ev)
+            if (e) (void)hipEventDestroy(e);
+        if (mem) (void)hipHostFree(mem);
+    }
+};
+
+std::mutex g_mu;
+std::vector<Staging*> g_idle;  // at most kMaxIdle
+
+// First touch of new pinned pages costs some 0.4 ms a MiB, so a set outlives the
+// call; concurrent calls each lease their own.
+Staging* lease()
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        for (size_t i = 0; i < g_idle.size(); ++i) {
+            if (g_idle[i]->dev != dev) continue;
+            Staging* s = g_idle[i];
+            g_idle.erase(g_idle.begin() + (long)i);
+            return s;
+        }
+    }
+    Staging* s = new (std::nothrow) Staging;
+    if (s && !s->create()) {
+        s->destroy();
+        delete s;
+        s = nullptr;
+    }
+    if (!s) (void)hipGetLastError();  // the caller takes the other way
+    return s;
+}
+
+void give_back(Staging* s)
+{
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        if ((int)g_idle.size() < kMaxIdle) {
+            try {
+                g_idle.push_back(s);
+                return;
+            } catch (const std::bad_alloc&) {
+            }
+        }
+    }
+    s->destroy();
+    delete s;
+}
+
+// One copy in pieces.  Piece c uses buffer c % kBuffers once piece c - kBuffers
+// has left it.  Threads take pieces in order, so of the pieces taken and not done
+// the lowest never waits for one that nobody works on.
+struct Copy {
+    Staging* s;
+    char* dev;
+    char* host;
+    size_t bytes;
+    bool up;  // to the device
+    long pieces;
+    std::atomic<long> next{0};
+    std::atomic<long> queued[kBuffers];  // pieces queued on the link so far, per buffer
+    std::atomic<bool> failed{false};
+
+    char* buffer(long c) const { return s->mem + (size_t)(c % kBuffers) * kPiece; }
+    size_t size(long c) const { return std::min(kPiece, bytes - (size_t)c * kPiece); }
+
+    // Queues piece c's transfer between its buffer and the device.
+    bool queue(long c)
+    {
+        const int b = (int)(c % kBuffers);
+        char* d = dev + (size_t)c * kPiece;
+        const hipError_t e = up ? hipMemcpyAsync(d, buffer(c), size(c), hipMemcpyHostToDevice, nullptr)
+                                : hipMemcpyAsync(buffer(c), d, size(c), hipMemcpyDeviceToHost, nullptr);
+        if (e != hipSuccess || hipEventRecord(s->ev[b], nullptr) != hipSuccess) return false;
+        queued[b].store(c / kBuffers + 1, std::memory_order_release);
+        return true;
+    }
+    // Until piece c's transfer is queued and over.
+    bool arrived(long c)
+    {
+        const int b = (int)(c % kBuffers);
+        while (queued[b].load(std::memory_order_acquire) <= c / kBuffers) {
+            if (failed.load(std::memory_order_relaxed)) return false;
+            std::this_thread::yield();
+        }
+        return hipEventSynchronize(s->ev[b]) == hipSuccess;
+    }
+    bool piece(long c)
+    {
+        char* h = host + (size_t)c * kPiece;
+        if (up) {
+            if (c >= kBuffers && !arrived(c - kBuffers)) return false;
+            std::memcpy(buffer(c), h, size(c));
+            return queue(c);
+        }
+        if (!arrived(c)) return false;
+        std::memcpy(h, buffer(c), size(c));
+        return c + kBuffers >= pieces || queue(c + kBuffers);
+    }
+    void work()
+    {
+        if (hipSetDevice(s->dev) != hipSuccess) failed.store(true);
+        for (;;) {
+            const long c = next.fetch_add(1, std::memory_order_relaxed);
+            if (c >= pieces || failed.load(std::memory_order_relaxed)) return;
+            if (!piece(c)) failed.store(true);
+        }
+    }
+};
+
+int staged(Staging* s, char* dev, char* host, size_t bytes, bool up)
+{
+    Copy c;
+    c.s = s;
+    c.dev = dev;
+    c.host = host;
+    c.bytes = bytes;
+    c.up = up;
+    c.pieces = (long)((bytes + kPiece - 1) / kPiece);
+    for (auto& q : c.queued) q.store(0);
+    if (!up) {
+        for (long i = 0; i < std::min<long>(kBuffers, c.pieces); ++i)
+            if (!c.queue(i)) c.failed.store(true);
+    }
+    std::thread th[kThreads - 1];
+    for (std::thread& t : th) {
+        try {
+            t = std::thread([&c] { c.work(); });
+        } catch (const std::exception&) {
+            break;  // fewer threads, the same pieces
+        }
+    }
+    c.work();
+    for (std::thread& t : th)
+        if (t.joinable()) t.join();
+    // the buffers are idle, and the data there, from here on
+    if (hipStreamSynchronize(nullptr) != hipSuccess) c.failed.store(true);
+    return c.failed.load() ? PERKS_ERR_HIP : PERKS_OK;
+}
+
+// Memory the runtime knows (pinned, managed) goes over the link as it is.
+bool pageable(const void* p)
+{
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return at.type == hipMemoryTypeUnregistered;
+}
+
+int copy(void* dev, void* host, size_t bytes, bool up)
+{
+    if (bytes >= kMinStaged && pageable(host)) {
+        if (Staging* s = lease()) {
+            const int rc = staged(s, (char*)dev, (char*)host, bytes, up);
+            give_back(s);
+            return rc;
+        }
+    }
+    const hipError_t e = up ? hipMemcpy(dev, host, bytes, hipMemcpyHostToDevice)
+                            : hipMemcpy(host, dev, bytes, hipMemcpyDeviceToHost);
+    return e == hipSuccess ? PERKS_OK : PERKS_ERR_HIP;
+}
+
+}  // namespace
+
+int copy_to_device(void* dst, const void* src, size_t bytes) { return copy(dst, const_cast<void*>(src), bytes, true); }
+int copy_to_host(void* dst, const void* src, size_t bytes) { return copy(const_cast<void*>(src), dst, bytes, false); }
+
+}  // namespace perks
