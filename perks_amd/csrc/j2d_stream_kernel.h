@@ -207,6 +207,14 @@ struct RowBuf<fmt::bf16s, true> : RowBuf16<fmt::bf16s, PERKS_BF16> {};
 // 64-bit addresses per row and level had some 20 scalar ones beside them, issued at
 // the same rate.
 //
+// At a face under the zero boundary a row's select covers side and bottom alike,
+// with no branch: the levels' rows are scheduled together.  Branches per level and
+// row, though hardly ever taken: 512 FP32 grids of 64 to 1024 rows and columns, 5
+// points, 12.9 ms, the select 11.7; 8192^2 FP32 9 points x 500 steps 29.8 and 28.2
+// ms; 6000^2 BF16 5 points 0.90 of the time.  (A second copy of the trip without
+// tests, for trips away from the faces, takes registers: 9 points at two workgroups
+// per CU instead of four, 31.0 ms.)
+//
 // And the loop has one way in, one back edge and the same memory operations on
 // both: the compiler's waits for the rows in flight are those of the steady
 // state.  With an exit or a conditional store between the rows it waited for
@@ -292,18 +300,13 @@ struct Strip {
         }
     }
 
-    // Lanes beyond a side face take the boundary value of their row.
+    // Lanes beyond a side face take the edge value of their row (clamp).
     __device__ __forceinline__ void side_faces(C (&v)[H]) const
     {
-        if constexpr (ZERO) {
+        const C vw = read_lane(v[0], lane_w);
+        const C ve = read_lane(v[H - 1], lane_e);
 #pragma unroll
-            for (int h = 0; h < H; ++h) v[h] = out ? (C)0 : v[h];
-        } else {
-            const C vw = read_lane(v[0], lane_w);
-            const C ve = read_lane(v[H - 1], lane_e);
-#pragma unroll
-            for (int h = 0; h < H; ++h) v[h] = out ? (x < 0 ? vw : ve) : v[h];
-        }
+        for (int h = 0; h < H; ++h) v[h] = out ? (x < 0 ? vw : ve) : v[h];
     }
 
     // Level LV1 = LV + 1 computes row q = i - R*LV1 from level LV's window.  The
@@ -334,17 +337,23 @@ struct Strip {
             if constexpr (LV1 == L) {
                 store((uint32_t)(q - ys) < (uint32_t)(ye - ys), v);
             } else {
-                if constexpr (EDGE) {
+                if constexpr (EDGE && ZERO) {
+                    // Lanes beyond a side face and rows beyond the others hold 0: one select
+                    // with a mask, and no branch between the levels' rows.
+                    const bool outside = out | ((uint32_t)q >= (uint32_t)ny);
+#pragma unroll
+                    for (int h = 0; h < H; ++h) v[h] = outside ? (C)0 : v[h];
+                } else if constexpr (EDGE) {
                     if (rarely(xedge)) {
                         keep_branch();
                         side_faces(v);
                     }
                     if (rarely((uint32_t)q >= (uint32_t)ny)) {
-                        // Rows below the bottom face read row ny-1 (clamp) or 0 (zero).
-                        // (Above the top one: 0, or row 0 once it is known, below.)
+                        // Rows below the bottom face read row ny-1.
+                        // (Above the top one: row 0 once it is known, below.)
                         keep_branch();
 #pragma unroll
-                        for (int h = 0; h < H; ++h) v[h] = ZERO ? (C)0 : win[LV1][mq(REL - 1)][BOX ? R : 0][h];
+                        for (int h = 0; h < H; ++h) v[h] = win[LV1][mq(REL - 1)][BOX ? R : 0][h];
                     }
                 }
                 keep(LV1, mq(REL), v);
