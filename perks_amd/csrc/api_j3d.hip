@@ -322,6 +322,7 @@ int perks_release(void)
     const int a = perks::release_persistent_scratch();
     const int b = perks::release_j2d_scratch();
     const int c = perks::release_cg_scratch();
+    perks::release_host_copy();
     return a != PERKS_OK ? a : (b != PERKS_OK ? b : c);
 }
 

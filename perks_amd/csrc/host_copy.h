@@ -10,5 +10,7 @@ namespace perks {
 // the data, when they return.  PERKS_OK or PERKS_ERR_HIP.
 int copy_to_device(void* dst, const void* src, size_t bytes);
 int copy_to_host(void* dst, const void* src, size_t bytes);
+// Frees the pinned buffers that no copy is using.
+void release_host_copy();
 
 }  // namespace perks

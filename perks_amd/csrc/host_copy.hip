@@ -33,7 +33,7 @@ constexpr size_t kPiece = (size_t)4 << 20;
 constexpr int kBuffers = 4;
 constexpr int kThreads = 4;                // with the caller's
 constexpr size_t kMinStaged = 2 * kPiece;  // below, there is nothing to overlap
-constexpr int kMaxIdle = 2;                // sets kept between calls (16 MiB each); more are freed on return
+constexpr int kMaxIdle = 2;                // sets kept between calls, until perks_release() (16 MiB each)
 
 // Pinned buffers of one copy, and an event per buffer.
 struct Staging {
@@ -225,6 +225,19 @@ int copy(void* dev, void* host, size_t bytes, bool up)
 }
 
 }  // namespace
+
+void release_host_copy()
+{
+    std::vector<Staging*> idle;
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        idle.swap(g_idle);
+    }
+    for (Staging* s : idle) {
+        s->destroy();
+        delete s;
+    }
+}
 
 int copy_to_device(void* dst, const void* src, size_t bytes) { return copy(dst, const_cast<void*>(src), bytes, true); }
 int copy_to_host(void* dst, const void* src, size_t bytes) { return copy(const_cast<void*>(src), dst, bytes, false); }

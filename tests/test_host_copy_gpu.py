@@ -43,3 +43,11 @@ def test_callers_at_once(gpu):
         t.join()
     for f, g in zip(fields, got):
         assert g.tobytes() == O.iterate(f, st, 3).tobytes()
+
+
+def test_release_between_calls(gpu):
+    field = O.uniform(9 * MIB // 4, 3, -1.0, 1.0, np.float32).reshape(1, 1, -1)
+    for _ in range(2):
+        got, _ = P.j3d_run(field, 0, method="plain", boundary="zero")
+        assert got.tobytes() == field.tobytes()
+        P.release()
