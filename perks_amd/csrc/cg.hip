@@ -124,7 +124,6 @@ struct CgArgs {
     const int32_t* rowptr;
     const int32_t* col;
     const V* val;
-    long long nnz;
     int ndiag;
     int32_t offs[kMaxDiag];
     // vectors
@@ -358,6 +357,7 @@ struct Lds {
     lds_ptr<V> mval;
     lds_ptr<int32_t> mcol;
     int mat;
+    int end;  // CSR: where the matrix's entries end (rowptr[n])
 };
 
 template <typename V, int FMT>
@@ -379,6 +379,9 @@ __device__ __forceinline__ Lds<V> lds_view(const CgArgs<V>& a, lds_ptr<unsigned 
     c.mval = reinterpret_cast<lds_ptr<V>>(dyn + off);
     off += (size_t)c.mat * (FMT == FMT_CSR ? 1 : a.ndiag) * sizeof(V);
     c.mcol = reinterpret_cast<lds_ptr<int32_t>>(dyn + off);
+    // from the row offsets, not the caller's nnz: an nnz that counts the arrays'
+    // capacity would let the last rows' wide loads pass the arrays' end
+    c.end = FMT == FMT_CSR ? a.rowptr[a.n] : 0;
     return c;
 }
 
@@ -635,7 +638,7 @@ __device__ __forceinline__ V row_value(const CgArgs<V>& a, const Lds<V>& c, int 
         const int k0 = valid ? a.rowptr[i] : 0;
         const int k1 = valid ? a.rowptr[i + 1] : 0;
         if constexpr (!MC) {
-            if (__ballot((long long)k1 + kCsrChunk > a.nnz) == 0)
+            if (__ballot(k1 > c.end - kCsrChunk) == 0)
                 return csr_short_from<true, V>(a.col, a.val, 0, k0, k1, c, kb, false, op);
             return csr_short_from<false, V>(a.col, a.val, 0, k0, k1, c, kb, false, op);
         }
@@ -1395,7 +1398,6 @@ int cg_solve(int fmt, const perks_csr* csr, const perks_dia* dia, const double* 
             a.rowptr = csr->rowptr;
             a.col = csr->col;
             a.val = csr->val;
-            a.nnz = csr->nnz;
         } else {
             a.val = dia->val;
             a.ndiag = dia->ndiag;
@@ -1510,7 +1512,6 @@ int cg_solve(int fmt, const perks_csr* csr, const perks_dia* dia, const double* 
             if (fmt == FMT_CSR) {
                 f.rowptr = csr->rowptr;
                 f.col = csr->col;
-                f.nnz = csr->nnz;
             } else {
                 f.ndiag = dia->ndiag;
                 for (int d = 0; d < dia->ndiag; ++d) f.offs[d] = dia->offsets[d];
@@ -1604,7 +1605,6 @@ int cg_solve_f32(int fmt, const perks_csr_f32* csr, const perks_dia_f32* dia, co
         f.rowptr = csr->rowptr;
         f.col = csr->col;
         f.val = csr->val;
-        f.nnz = csr->nnz;
     } else {
         f.ndiag = dia->ndiag;
         for (int d = 0; d < dia->ndiag; ++d) f.offs[d] = dia->offsets[d];
