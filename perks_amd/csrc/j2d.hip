@@ -34,6 +34,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -207,49 +208,98 @@ RowCut cut_rows(int ny, int seg, int edge)
 
 // Rows per segment of the streaming kernel: the height that makes a pass
 // shortest, among those whose rows (seg + 2RL with the ghost rows) fill whole
-// trips of stream_trip(R) rows.
-//   Persistent: the resident waves take as many rounds as the items need, each
-//   of a segment's rows and the time until its first loads have arrived (about
-//   2 us, which is 150 / (L * points) rows' arithmetic).  8192^2 FP32 2d9pt, 4
-//   steps per pass: one round of 154 rows, 29.4 ms for 500 steps; four rounds of
-//   37 rows take 31.1.
-//   Per step: a CU's workgroups run together and share its bandwidth, so what
-//   counts is the rows of the CU that gets most, two rows' time for starting
-//   each item, and that one workgroup alone hides no latency.  2048^2 FP64
-//   2d5pt: 25 rows (3 workgroups per CU) 13.0 us per step, 43 rows (2) 13.5,
-//   16 rows (5) 16.8, 7 rows (10) 16.0.
-int stream_segment(const J2dSpec* specs, int n, int R, int npts, int L, int VW, int edge, bool plain,
-                   const Resident& res)
+// trips of stream_trip(R) rows.  A pass, in units of one wave's row of the
+// update's arithmetic (`ops` per row and lane), by the waves that the fullest
+// SIMD runs (one at a time, or all that are resident in a round) and the rows of
+// an item:
+//   waves * (rows + h)    what the SIMD issues, starting an item h rows' worth;
+//   rounds * f / ops      until the first loads of a round have arrived;
+//   e * rows              what the slowest wave takes longer than the others:
+//                         persistent 0.37, under clamp with two or more levels
+//                         0.86 more (the strips at a side face read lanes and
+//                         branch); per step 9 / ops, and half its rows where it
+//                         is alone on its SIMD and hides no latency.
+// Per step, fields beyond the last-level cache read memory in more open rows the
+// taller the segments, unless arithmetic hides it: 8000^2 FP32 9-point 16 to 34
+// rows 102-109 us a step, 97 rows 116, 124 rows 124.
+// Fitted to 2040 combinations of shapes, formats, roundings, boundaries, methods
+// and sizes from 64^2 to 8000^2 at 5 to 20 heights each: 1.2% (per step) and 1.6%
+// (persistent) more time than the best of those heights, geometric mean.  us for
+// 24 steps by height:
+//   FP64 5 points 2048^2 per step: 7 rows 356, 16 482, 25 333, 52 362, 97 375
+//   BF16 stochastic 9 points (radius 2) 2048^2 clamp per step: 6 rows 289, 16 299, 36 362
+//   FP16 25 points 2048^2, 2 steps per pass: 12 rows 500, 22 444, 32 536, 72 634
+struct PassCost {
+    bool plain, tall_dear;
+    int cus, occ;
+    double h, f, e, lone, ops;
+    int trip;
+    double operator()(long long items, double rows) const
+    {
+        const long long simds = 4LL * cus;
+        double w = std::ceil((double)((items + kStreamWaves - 1) / kStreamWaves) / cus);
+        double rounds;
+        if (plain) {
+            rounds = std::max(1.0, w / occ);
+        } else {
+            rounds = (double)((items + simds * occ - 1) / (simds * occ));
+            if (rounds > 1) w = rounds * occ;
+        }
+        double c = w * (rows + h) + rounds * f / ops + (e + (w == 1 ? lone : 0.0)) * rows;
+        if (tall_dear) c *= 1 + std::max(0.0, 3.7 / ops - 0.07) * std::log(std::max(1.0, rows / trip));
+        return c;
+    }
+};
+
+constexpr double kLastLevelCache = 256.0 * (1 << 20);  // bytes
+
+int stream_segment(const J2dSpec* specs, int n, int dtype, const ShapeDesc& sd, int L, int VW, bool pair, int edge,
+                   const perks_stencil_opts* o, const Resident& res)
 {
-    const int trip = stream_trip(R), ghost = 2 * R * L;
-    const int fill = 150 / (L * npts);
+    const int R = sd.radius, trip = stream_trip(R), ghost = 2 * R * L;
+    int npts = 0;
+    for (int g = 0; g < sd.ngroups; ++g) npts += sd.g[g].npts;
+    PassCost cost;
+    cost.plain = o->method == PERKS_METHOD_PLAIN;
+    cost.cus = res.cus;
+    cost.occ = res.occ;
+    cost.trip = trip;
+    cost.ops = (double)L * npts * (pair ? 2 : 1);
+    cost.h = cost.plain ? 0.55 + 33.3 / cost.ops : 1.2;
+    cost.f = cost.plain ? 250 : 100;
+    cost.e = cost.plain ? 9 / cost.ops : (o->boundary == PERKS_BC_CLAMP && L > 1 ? 1.23 : 0.37);
+    cost.lone = cost.plain ? 0.53 : 0.0;
+    // The grids by passes, longest first: as many run in pass p as have more than p.
+    struct Run {
+        int passes, nx, ny;
+    };
+    std::vector<Run> runs;
+    double bytes = 0;
     int most = 1;
-    for (int i = 0; i < n; ++i)
-        if (specs[i].steps > 0) most = std::max(most, specs[i].ny);
+    for (int i = 0; i < n; ++i) {
+        if (specs[i].steps <= 0) continue;
+        runs.push_back({n == 1 ? 1 : (specs[i].steps + L - 1) / L, specs[i].nx, specs[i].ny});
+        bytes += 2.0 * specs[i].nx * specs[i].ny * (dtype == PERKS_F64 ? 8 : (dtype == PERKS_F32 ? 4 : 2));
+        most = std::max(most, specs[i].ny);
+    }
+    std::sort(runs.begin(), runs.end(), [](const Run& a, const Run& b) { return a.passes > b.passes; });
+    cost.tall_dear = cost.plain && bytes > kLastLevelCache;
     int best = 1;
     double best_cost = 1e300;
     // (a coarser walk over the heights of a batch: its grids average them out)
     for (long long k = ghost / trip + 1;; k += 1 + k / (n == 1 ? 16 : 4)) {
         const int seg = (int)std::min<long long>(k * trip - ghost, 0x7fffffffLL);
-        long long items = 0, passes = 1;  // over all passes
-        for (int i = 0; i < n; ++i) {
-            if (specs[i].steps <= 0) continue;
-            const long long np = n == 1 ? 1 : (specs[i].steps + L - 1) / L;
-            items += (specs[i].nx + VW - 1LL) / VW * cut_rows(specs[i].ny, seg, edge).count(specs[i].ny) * np;
-            passes = std::max(passes, np);
+        long long items = 0;
+        double rows = 0, total = 0;  // rows of the items so far, and of the passes
+        for (size_t i = 0; i < runs.size(); ++i) {
+            const long long c = (runs[i].nx + VW - 1LL) / VW * cut_rows(runs[i].ny, seg, edge).count(runs[i].ny);
+            items += c;
+            rows += (double)c * (std::min(seg, runs[i].ny) + ghost);
+            const int next = i + 1 < runs.size() ? runs[i + 1].passes : 0;
+            if (runs[i].passes > next) total += (double)(runs[i].passes - next) * cost(items, rows / (double)items);
         }
-        double cost;
-        if (plain) {
-            const long long per_pass = 4LL * res.cus * passes;
-            const double wgs = (double)((items + per_pass - 1) / per_pass);
-            cost = (wgs + 0.5) * ((double)seg + ghost + 2);
-        } else {
-            // half a round is lost at the end of each pass of several grids
-            const double rounds = (double)((items + res.waves() - 1) / res.waves()) + (n == 1 ? 0.0 : 0.5 * passes);
-            cost = rounds * ((double)seg + ghost + fill);
-        }
-        if (cost < best_cost * (1 - 1e-9)) {
-            best_cost = cost;
+        if (total < best_cost * (1 - 1e-9)) {
+            best_cost = total;
             best = seg;
         }
         if (seg >= most) break;
@@ -257,8 +307,8 @@ int stream_segment(const J2dSpec* specs, int n, int R, int npts, int L, int VW, 
     return best;
 }
 
-int build_work(const J2dSpec* specs, int n, const ShapeDesc& sd, int tx, int ty, int L, bool plain,
-               const Resident& res, Work* w)
+int build_work(const J2dSpec* specs, int n, int dtype, const ShapeDesc& sd, int tx, int ty, int L,
+               const perks_stencil_opts* o, const Resident& res, Work* w)
 {
     const int R = sd.radius;
     const bool stream = ty == 0;
@@ -267,11 +317,9 @@ int build_work(const J2dSpec* specs, int n, const ShapeDesc& sd, int tx, int ty,
     if (VW < 1 || (!stream && VH < 1)) return PERKS_ERR_INVALID_ARG;
     const int edge = 2 * R * L + 1;  // fewest rows of a strip's first and last segment
     if (stream) {
-        int npts = 0;
-        for (int g = 0; g < sd.ngroups; ++g) npts += sd.g[g].npts;
         for (int i = 0; i < n; ++i)
             if (specs[i].ny <= 0 || specs[i].nx <= 0) return PERKS_ERR_INVALID_ARG;
-        VH = stream_segment(specs, n, R, npts, L, VW, edge, plain, res);
+        VH = stream_segment(specs, n, dtype, sd, L, VW, tx == 128, edge, o, res);
     }
     std::vector<int> order(n);
     for (int i = 0; i < n; ++i) order[i] = i;
@@ -479,7 +527,7 @@ int j2d_run(int dtype, J2dSpec* specs, int n, const perks_stencil_opts* o, hipSt
     Resident res;
     rc = resident(dtype, o, cf, c, &res);
     if (rc != PERKS_OK) return rc;
-    rc = build_work(specs, n, *sd, tx, ty, c.levels, o->method == PERKS_METHOD_PLAIN, res, &w);
+    rc = build_work(specs, n, dtype, *sd, tx, ty, c.levels, o, res, &w);
     if (rc != PERKS_OK) return rc;
     for (int i = 0; i < n; ++i) specs[i].result_in_b = w.result_in_b[i];
     if (w.grids.empty()) {
@@ -584,7 +632,7 @@ int j2d_run_noalloc(int dtype, J2dSpec* specs, int n, const perks_stencil_opts* 
     Resident res;
     rc = resident(dtype, o, cf, c, &res);
     if (rc != PERKS_OK) return rc;
-    rc = build_work(specs, n, *sd, tx, ty, c.levels, o->method == PERKS_METHOD_PLAIN, res, &w);
+    rc = build_work(specs, n, dtype, *sd, tx, ty, c.levels, o, res, &w);
     if (rc != PERKS_OK) return rc;
     if (w.grids.size() > (size_t)PERKS_NOALLOC_MAX_GRIDS || w.active.size() > (size_t)PERKS_NOALLOC_MAX_PASSES) {
         std::fprintf(stderr,
@@ -697,8 +745,8 @@ double time_config(int dtype, const perks_stencil_opts* o, const KCoefs& cf, con
     Work w;
     Resident res;
     if (resident(dtype, o, cf, c, &res) != PERKS_OK) return 0.0;
-    if (build_work(specs.data(), (int)specs.size(), sd, tx, ty, c.levels, o->method == PERKS_METHOD_PLAIN, res,
-                   &w) != PERKS_OK || w.grids.empty())
+    if (build_work(specs.data(), (int)specs.size(), dtype, sd, tx, ty, c.levels, o, res, &w) != PERKS_OK ||
+        w.grids.empty())
         return 0.0;
     DeviceWork dw;
     double best = 0.0;
@@ -816,8 +864,7 @@ int plan_batch(int dtype, const perks_grid2d* grids, int ngrids, const perks_ste
     Resident res;
     rc = resident(dtype, o, cf, p->cfg, &res);
     if (rc == PERKS_OK)
-        rc = build_work(specs.data(), ngrids, *sd, tx, ty, p->cfg.levels, o->method == PERKS_METHOD_PLAIN, res,
-                        &p->work);
+        rc = build_work(specs.data(), ngrids, dtype, *sd, tx, ty, p->cfg.levels, o, res, &p->work);
     if (rc == PERKS_OK) rc = p->dw.upload(p->work, stream);
     if (rc == PERKS_OK) prepare_launch(dtype, o, cf, p->cfg, res, p->work, p->dw, p->gs, &p->launch);
     if (rc == PERKS_OK && hipStreamSynchronize(stream) != hipSuccess) rc = PERKS_ERR_HIP;

@@ -198,10 +198,11 @@ struct RowBuf<fmt::bf16s, true> : RowBuf16<fmt::bf16s, PERKS_BF16> {};
 // reach row 0 or past the last one.
 //
 // A level computes a row as soon as the row it needs last arrives, without
-// asking whether the others have: the first R*l rows of a segment come out of a
-// window that does not hold their inputs yet, as values that no stored row
-// reads.  Every row also stores, where there is nothing to store to a descriptor of
-// size 0.  So away from the faces a row costs its update and some 15 scalar
+// asking whether it is wanted: what a segment's rows are is known by position
+// only.  In the first trip of a segment level l starts at stage 2R*l, fixed at
+// compile time, as its window is whole from there on (trips are longer than
+// 2R*L rows).  Every stage stores, where there is nothing to store to a descriptor
+// of size 0.  So away from the faces a row costs its update and some 15 scalar
 // operations, whatever the depth of the pass.  The 5-point star in FP32 has 9
 // vector operations per row and level; the form with range and face tests and
 // 64-bit addresses per row and level had some 20 scalar ones beside them, issued at
@@ -214,6 +215,15 @@ struct RowBuf<fmt::bf16s, true> : RowBuf16<fmt::bf16s, PERKS_BF16> {};
 // ms; 6000^2 BF16 5 points 0.90 of the time.  (A second copy of the trip without
 // tests, for trips away from the faces, takes registers: 9 points at two workgroups
 // per CU instead of four, 31.0 ms.)
+//
+// A segment of one trip (per step: the small ones) runs a form of its own, which
+// requests no further rows and stores none but its own: on the smallest launches a
+// CU's memory instructions count, not its arithmetic.  With every trip alike, 16-bit
+// fields paid the hash and the rounding for 2R*L more rows a segment and level, and
+// a short segment twice its memory instructions.  us for 100 steps, every trip
+// alike -> here: BF16 stochastic 9 points (radius 2) 2048^2 clamp, one step per
+// launch 1535 -> 1144, 5 points 8000 x 200 807 -> 637; FP16 25 points 2048^2 zero,
+// two per pass 2388 -> 1644.
 //
 // And the loop has one way in, one back edge and the same memory operations on
 // both: the compiler's waits for the rows in flight are those of the steady
@@ -233,6 +243,10 @@ struct Strip {
     static constexpr int UF = D;              // rows per loop trip, so every ring slot is static
     static constexpr int NS = BOX ? Q : 1;    // boxes keep the x shifts of a row
     static constexpr int H = PAIR ? 2 : 1;    // columns per lane
+
+    // A segment's first trip of several, the ones after it, and the trip of a
+    // segment that has one.
+    enum { FIRST, LATER, ONLY };
 
     const S* src;
     S* dst;
@@ -311,10 +325,14 @@ struct Strip {
 
     // Level LV1 = LV + 1 computes row q = i - R*LV1 from level LV's window.  The
     // slot it writes held row q - Q, which no level needs any more.
-    template <int U, int LV>
+    template <int TRIP, int U, int LV>
     __device__ __forceinline__ void level(int i)
     {
-        if constexpr (LV < L) {
+        if constexpr (TRIP != LATER && LV < L && U < 2 * R * (LV + 1)) {
+            const C none[H] = {};
+            if constexpr (TRIP == FIRST) store(false, none);
+            else sp += row_bytes;
+        } else if constexpr (LV < L) {
             constexpr int LV1 = LV + 1;
             constexpr int REL = U - R * LV1;  // relative index of row q
             const int q = i - R * LV1;
@@ -371,44 +389,41 @@ struct Strip {
                     }
                 }
             }
-            level<U, LV + 1>(i);
+            level<TRIP, U, LV + 1>(i);
         }
     }
 
     // Iteration i (stage U = (i - i0) mod UF): level-0 row i, loaded D
     // iterations ago, enters the window, and row i + D is requested into its
     // in-flight slot.
-    template <int U>
+    template <int TRIP, int U>
     __device__ __forceinline__ void stage(int i)
     {
         const Raw w = fl[U];
-        fl[U] = next_row();  // issued before row i is waited for
+        if constexpr (TRIP != ONLY) fl[U] = next_row();  // issued before row i is waited for
         C v[H];
         Row::unpack(w, v);
         if constexpr (EDGE && PAIR && !ZERO) {
-            if (rarely(xedge)) {
-                // a pair beyond a side face loaded the edge pair: both halves take the edge column
-                keep_branch();
-                const C a = v[0], b = v[1];
-                v[0] = x > nx - 2 ? b : a;
-                v[1] = x < 0 ? a : b;
-            }
+            // a pair beyond a side face loaded the edge pair: both halves take the edge column
+            const C a = v[0], b = v[1];
+            v[0] = x > nx - 2 ? b : a;
+            v[1] = x < 0 ? a : b;
         }
         keep(0, mq(U), v);
-        level<U, 0>(i);
+        level<TRIP, U, 0>(i);
     }
 
     // One trip.  Rows past the segment's last are computed and not stored
     // (segments are cut to whole trips where they can be, cut_rows in j2d.hip).
-    template <int U = 0>
+    template <int TRIP, int U = 0>
     __device__ __forceinline__ void trip(int i)
     {
         if constexpr (U < UF) {
-            stage<U>(i);
+            stage<TRIP, U>(i);
             // Rows are scheduled one by one: mixed, their values take up to
             // 50% more registers.
             __builtin_amdgcn_sched_barrier(0);
-            trip<U + 1>(i + 1);
+            trip<TRIP, U + 1>(i + 1);
         }
     }
 
@@ -431,24 +446,17 @@ struct Strip {
         lrow = i0;
         lend = min(iend, ny - 1);
         lp = reinterpret_cast<const char*>(src + (size_t)max(i0, 0) * nx + xb);
-        // the row that iteration i0 stores, D rows further for the ones dropped below
-        sp = reinterpret_cast<char*>(dst + xb) + (ptrdiff_t)(i0 - R * L - D) * (ptrdiff_t)row_bytes;
+        sp = reinterpret_cast<char*>(dst + xb) + (ptrdiff_t)(i0 - R * L) * (ptrdiff_t)row_bytes;
 #pragma unroll
-        for (int l = 0; l < L; ++l)
-#pragma unroll
-            for (int q = 0; q < Q; ++q)
-#pragma unroll
-                for (int t = 0; t < NS; ++t)
-#pragma unroll
-                    for (int h = 0; h < H; ++h) win[l][q][t][h] = (C)0;
-        // The rows in flight, each followed by a dropped store as in the loop.
-        const C none[H] = {};
-#pragma unroll
-        for (int t = 0; t < D; ++t) {
-            fl[t] = next_row();
-            store(false, none);
+        for (int t = 0; t < D; ++t) fl[t] = next_row();
+        if constexpr (L == 1) {
+            if (iend < i0 + UF) {
+                trip<ONLY>(i0);
+                return;
+            }
         }
-        for (int i = i0; i <= iend; i += UF) trip(i);
+        trip<FIRST>(i0);
+        for (int i = i0 + UF; i <= iend; i += UF) trip<LATER>(i);
     }
 };
 
