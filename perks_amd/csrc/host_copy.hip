@@ -27,24 +27,23 @@ namespace perks {
 
 namespace {
 
-// 17 us of the link go by between two pieces: 64 MiB in pieces of 1, 2 and 4 MiB
-// take 2.16, 1.73 and 1.55 ms; 8 buffers or threads, the same.
-constexpr size_t kPiece = (size_t)4 << 20;
-constexpr int kBuffers = 4;
-constexpr int kThreads = 4;                // with the caller's
-constexpr size_t kMinStaged = 2 * kPiece;  // below, there is nothing to overlap
-constexpr int kMaxIdle = 2;                // sets kept between calls, until perks_release() (16 MiB each)
+constexpr int kBuffers = kStagingBuffers;
+constexpr int kThreads = 3;                     // with the caller's; 4 or 8, the same
+constexpr size_t kMinStaged = (size_t)8 << 20;  // below, there is too little to overlap
+constexpr int kMaxIdle = 2;  // sets kept between calls, until perks_release() (12 to 36 MiB each)
 
 // Pinned buffers of one copy, and an event per buffer.
 struct Staging {
     int dev = -1;
+    size_t cap = 0;  // bytes of a buffer
     char* mem = nullptr;
     hipEvent_t ev[kBuffers] = {};
 
-    bool create()
+    bool create(size_t bytes)
     {
+        cap = staging_capacity(bytes);
         if (hipGetDevice(&dev) != hipSuccess) return false;
-        if (hipHostMalloc((void**)&mem, kPiece * kBuffers, hipHostMallocDefault) != hipSuccess) {
+        if (hipHostMalloc((void**)&mem, cap * kBuffers, hipHostMallocDefault) != hipSuccess) {
             mem = nullptr;
             return false;
         }
@@ -69,7 +68,7 @@ std::vector<Staging*> g_idle;  // at most kMaxIdle
 
 // First touch of new pinned pages costs some 0.4 ms a MiB, so a set outlives the
 // call; concurrent calls each lease their own.
-Staging* lease()
+Staging* lease(size_t bytes)
 {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return nullptr;
@@ -83,7 +82,7 @@ Staging* lease()
         }
     }
     Staging* s = new (std::nothrow) Staging;
-    if (s && !s->create()) {
+    if (s && !s->create(bytes)) {
         s->destroy();
         delete s;
         s = nullptr;
@@ -117,19 +116,20 @@ struct Copy {
     char* host;
     size_t bytes;
     bool up;  // to the device
+    size_t piece_bytes;
     long pieces;
     std::atomic<long> next{0};
     std::atomic<long> queued[kBuffers];  // pieces queued on the link so far, per buffer
     std::atomic<bool> failed{false};
 
-    char* buffer(long c) const { return s->mem + (size_t)(c % kBuffers) * kPiece; }
-    size_t size(long c) const { return std::min(kPiece, bytes - (size_t)c * kPiece); }
+    char* buffer(long c) const { return s->mem + (size_t)(c % kBuffers) * s->cap; }
+    size_t size(long c) const { return std::min(piece_bytes, bytes - (size_t)c * piece_bytes); }
 
     // Queues piece c's transfer between its buffer and the device.
     bool queue(long c)
     {
         const int b = (int)(c % kBuffers);
-        char* d = dev + (size_t)c * kPiece;
+        char* d = dev + (size_t)c * piece_bytes;
         const hipError_t e = up ? hipMemcpyAsync(d, buffer(c), size(c), hipMemcpyHostToDevice, nullptr)
                                 : hipMemcpyAsync(buffer(c), d, size(c), hipMemcpyDeviceToHost, nullptr);
         if (e != hipSuccess || hipEventRecord(s->ev[b], nullptr) != hipSuccess) return false;
@@ -148,7 +148,7 @@ struct Copy {
     }
     bool piece(long c)
     {
-        char* h = host + (size_t)c * kPiece;
+        char* h = host + (size_t)c * piece_bytes;
         if (up) {
             if (c >= kBuffers && !arrived(c - kBuffers)) return false;
             std::memcpy(buffer(c), h, size(c));
@@ -177,7 +177,8 @@ int staged(Staging* s, char* dev, char* host, size_t bytes, bool up)
     c.host = host;
     c.bytes = bytes;
     c.up = up;
-    c.pieces = (long)((bytes + kPiece - 1) / kPiece);
+    c.piece_bytes = staging_piece(s->cap, bytes);
+    c.pieces = (long)((bytes + c.piece_bytes - 1) / c.piece_bytes);
     for (auto& q : c.queued) q.store(0);
     if (!up) {
         for (long i = 0; i < std::min<long>(kBuffers, c.pieces); ++i)
@@ -213,7 +214,7 @@ bool pageable(const void* p)
 int copy(void* dev, void* host, size_t bytes, bool up)
 {
     if (bytes >= kMinStaged && pageable(host)) {
-        if (Staging* s = lease()) {
+        if (Staging* s = lease(bytes)) {
             const int rc = staged(s, (char*)dev, (char*)host, bytes, up);
             give_back(s);
             return rc;
