@@ -149,9 +149,15 @@ static Split split_domain(const Variant& v, int nz, int ny, int nx, int bc, int 
 // Microseconds of one pass of `l` levels: a barrier and a fill, and planes at a
 // rate per level of the format's update (with the boundary step of tiles that
 // have ghost lanes beyond an x face: always under clamp, on narrow grids under
-// zero) -- and, where the fields exceed the last-level cache, the traffic with
-// it.  Fitted to passes of 2, 3 and 4 levels over 26 domains from 32^3 to 512^3,
-// odd and flat ones among them, in five formats and both boundaries.
+// zero) -- and with it the traffic: from memory where the fields exceed the
+// last-level cache, from that cache what is beyond the L2s' share.  (Without the
+// latter two levels looked best on flat domains, whose passes move much for their
+// planes: FP64 clamp 50 x 512^2, 24 steps, equal weights 628 us at two levels, 567 at
+// four; contracted 612 and 523.)  The rates of the update forms -- gold order,
+// shared products, contracted -- differ, but levels and tile that one pays for do
+// for the others.  Fitted to passes of 2, 3 and 4 levels over 26 domains from 32^3
+// to 512^3, odd and flat ones among them, in five formats and both boundaries; the
+// traffic term to the choices below.
 static double pass_us(int dtype, bool sr, int bc, int nx, double cells, double planes, int l, double width)
 {
     const bool clamp = bc == PERKS_BC_CLAMP;
@@ -162,10 +168,10 @@ static double pass_us(int dtype, bool sr, int bc, int nx, double cells, double p
     default: a = sr ? (clamp ? 0.75 : 0.52) : (clamp ? 0.549 : 0.321); break;
     }
     if (!clamp && !j3dp::x_face_tiles(bc, nx, l)) a *= 1.266;
-    double t = 6.87 + planes * width * a * (l + (clamp ? 0.073 : 0.41));
+    const double t = 6.87 + planes * width * a * (l + (clamp ? 0.073 : 0.41));
     const double bytes = 2.0 * cells * elem_bytes(dtype);
-    if (bytes > 270e6) t = std::sqrt(t * t + bytes / 4.43e6 * (bytes / 4.43e6));
-    return t;
+    const double traffic = bytes > 270e6 ? bytes / 4.43e6 : std::max(0.0, bytes - 40e6) / 4e6;
+    return std::sqrt(t * t + traffic * traffic);
 }
 // ... and of `steps` steps in passes of up to L (0: of many, per step).
 static double run_us(int dtype, bool sr, int bc, int nx, double cells, const Split& s, int steps, int L,
@@ -182,9 +188,10 @@ static double run_us(int dtype, bool sr, int bc, int nx, double cells, const Spl
 // planes beside the 2L it reads beyond them is faster with fewer levels; in FP32
 // arithmetic a plane of the 16 x 2-row workgroup takes 0.59 of the 16 x 4 one's
 // time, which pays until the chip is full; and tile and round counts jump with
-// the sides.  The default stays unless the model finds 4% in a change.  Over
-// the combinations above at 24, 20 and 10 steps: 9% less time (geometric mean),
-// none more than 2% slower.  us for 24 steps, 4 levels (16-bit clamp: 3) of variant 0 -> chosen:
+// the sides.  The default stays unless the model finds 4% in a change.  24 steps of
+// 74 domains with sides from 24 to 700, six formats and roundings, both boundaries,
+// three update forms (2072 combinations): 10.7% more speed (geometric mean), none
+// more than 1% slower.  us, 4 levels (16-bit clamp: 3) of variant 0 -> chosen:
 //   FP64 zero 64^3 130 -> 109 (3 levels), 256^3 618 -> 553 (3), 260 x 61 x 700 645 -> 381 (3)
 //   FP32 clamp 64^3 137 -> 102, 128^3 190 -> 156 (variant 3, 4 levels), 150 x 250 x 350 429 -> 340 (2 levels)
 //   BF16 stochastic 128^3 219 -> 177 (variant 3)
@@ -412,6 +419,7 @@ int run_persistent_fmt(int dtype, void* d_a, void* d_b, int nz, int ny, int nx, 
         rep->result_in_b = npass % 2;
         rep->reserved[0] = a.levels;
         rep->reserved[1] = npass;
+        rep->reserved[2] = var;
     }
     return PERKS_OK;
 }

@@ -410,6 +410,7 @@ int run_resident(int dtype, void* d_a, void* d_b, int nz, int ny, int nx, int st
         rep->result_in_b = steps % 2;
         rep->reserved[0] = 1;
         rep->reserved[1] = steps;
+        rep->reserved[2] = kResidentVariant;
     }
     return PERKS_OK;
 }
