@@ -102,15 +102,22 @@ typedef struct perks_stencil_opts {
     /* experimental knobs, 0 = automatic:
      *   tune[0] plain: z-chunk per workgroup       tune[1] plain: 2 = cached stores (default nontemporal)
      *   tune[2] persistent: time steps per pass     tune[3] persistent: workgroups per CU
-     *           (3D 7-point default: 4; under the clamp boundary 3 for FP16 and for BF16
-     *           with nearest rounding; perks_j3d_autotune measures every choice)
+     *           (3D 7-point: where tune[2], [4] and [7] are all 0, two to four and the tile
+     *           variant by the domain, the format, the boundary and the number of steps;
+     *           report.reserved[0] and [2] say which ran, and report.result_in_b follows the
+     *           number of passes.  perks_j3d_autotune measures every choice)
      *   tune[4] tile variant.  3D 7-point persistent: 0..3 (rows x waves of its kernel;
-     *           FP64 0 = 12 waves x 3 rows, 3 = 8 waves x 5 rows), 4 = two columns per lane (FP32/FP16/BF16, even
+     *           FP64 0 = 12 waves x 3 rows, 3 = 8 waves x 5 rows; FP32 arithmetic 0 = 16 x 4,
+     *           3 = 16 x 2), 4 = two columns per lane (FP32/FP16/BF16, even
      *           widths) or, for FP64, 8 waves x 4 rows; 5 = resident tiles (FP64/FP32): the whole domain held
      *           in VGPRs across every step, one grid barrier per step, halos only through
      *           memory; PERKS_ERR_UNSUPPORTED_SIZE above perks_j3d_min_height's height.
      *           3D other shapes: 0 = default, 2 = register streaming (64 x 8 tiles),
-     *           4 = register streaming (64 x 16 tiles), 3 = LDS planes.
+     *           4 = register streaming (64 x 16 tiles), 3 = LDS planes.  The default is 2, but
+     *           for the 17- and 27-point shapes one step plane by plane (62 x 4 tiles) up to a
+     *           size of the fields that depends on format and method, and persistently with
+     *           more than one workgroup per CU or 300000 cells; 2 with tune[2] = 1 is that
+     *           form as well, up to the same size.
      *           2D: 0 = default (4 where it applies, else 2), 1 = LDS tile 128x64 (64x64 FP64),
      *           2 = row streaming through registers, one column per lane, 3 = LDS tile 128x32
      *           (64x32 FP64), 4 = row streaming, two columns per lane (FP32/FP16/BF16 storage,
@@ -177,7 +184,8 @@ typedef struct perks_plan_info {
 const char* perks_version(void);
 const char* perks_error_string(int code);
 int perks_query_device(int device, perks_device_caps* caps);
-/* Frees cached device scratch of the current device. */
+/* Frees cached device scratch of the current device, and the pinned host buffers
+ * that the host-array calls keep and no call is using. */
 int perks_release(void);
 
 /* ---- shapes --------------------------------------------------------------- */
@@ -189,6 +197,8 @@ int perks_shape_info(int shape, int32_t* dims, int32_t* radius, int32_t* ngroups
                      double* divisor, int32_t* npts, int32_t* prod_f64, int8_t* offsets);
 
 /* ---- planning (host only when caps != NULL) ------------------------------ */
+/* What a run of many steps uses: tile, steps per pass, slabs, grid.  A run knows its
+ * number of steps and may take others for few (see tune[2]). */
 int perks_j3d_plan(int dtype, int height, int width_y, int width_x, const perks_stencil_opts* opts,
                    const perks_device_caps* caps, int occupancy_hint, perks_plan_info* out);
 /* j3d_iterative(..., getminHeight=true): the largest height whose domain the
@@ -306,7 +316,7 @@ int perks_jacobi2d_batch(int dtype, perks_grid2d* grids, int ngrids, const perks
  * reference: it is for callers that cannot allocate device memory (tight
  * serving loops, harnesses that forbid hipMalloc).  The launch's scratch --
  * grid-barrier block, work list, per-pass active counts -- lives in a fixed
- * device array (about 0.9 MiB) that each GPU holds until the process ends,
+ * device array (about 0.5 MiB) that each GPU holds until the process ends,
  * so a batch may hold at most PERKS_NOALLOC_MAX_GRIDS grids with steps and
  * PERKS_NOALLOC_MAX_PASSES passes (per-step method: time steps) of its
  * longest grid; larger batches return PERKS_ERR_UNSUPPORTED_SIZE.  Calls on

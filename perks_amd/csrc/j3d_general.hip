@@ -12,7 +12,9 @@
 // its plane-by-plane form, j3d_sweep_kernel.h, up to the sizes of sweep_limit)
 // and the LDS-plane kernel (j3d_general_kernel.h; a workgroup per 64 x 16/32
 // tile, planes in LDS).
-// opts->tune[4] picks one: 2 = streaming, 3 = LDS planes, 0 = default.
+// opts->tune[4] picks one: 2 = streaming on 64 x 8 tiles, 4 = on 64 x 16 tiles,
+// 3 = LDS planes, 0 = default.  One step per pass (tune[2] = 1) of 2 is the
+// plane-by-plane form as far as the default takes it: the autotuner times both.
 #include "j3d_general.h"
 
 #include <algorithm>
@@ -108,14 +110,31 @@ size_t sweep_limit(int dtype, int shape, int method)
     return SIZE_MAX;
 }
 
-// The plane-by-plane form runs the shapes whose table allows it, at one step per
-// pass, in place of the short tile.  A persistent grid held to one workgroup per
-// CU keeps the two-step kernel, and with it the plan reported for that limit.
-bool use_sweep(int dtype, int shape, const perks_stencil_opts* o, int levels, size_t cells)
+// A persistent grid of one workgroup per CU takes the two-step windowed kernel up to
+// this many cells: it meets at half as many barriers, and so small a domain gives
+// the other form nothing to overlap them with.  us for 20 steps at one workgroup per
+// CU, windowed and plane by plane: FP32 17 points 48^3 131, 150, 64^3 153, 172, 72^3
+// 176, 179, 80^3 194, 181; FP64 27 points 48^3 168, 182, 64^3 199, 204, 72^3 239, 230,
+// 80^3 269, 222, 256^3 2312, 1115.
+constexpr size_t kLoneWindowedCells = 300000;
+
+// Whether a run takes the plane-by-plane form, at one step per pass: shapes whose
+// table allows it, up to sweep_limit, where the caller leaves the tile open or asks
+// for one step per pass of the streaming kernel.  `lone`: the persistent grid has
+// one workgroup per CU.
+bool use_sweep(int dtype, int shape, const perks_stencil_opts* o, size_t cells, bool lone)
 {
-    if (o->method != PERKS_METHOD_PLAIN && (o->blkpsm == 1 || o->tune[3] == 1)) return false;
-    return levels == 1 && (o->tune[4] == 0 || o->tune[4] == 2) && j3z::sweeps(shape) &&
-           2 * cells * elem_size(dtype) <= sweep_limit(dtype, shape, o->method);
+    const bool plain = o->method == PERKS_METHOD_PLAIN;
+    if (o->tune[4] != 0 && !(o->tune[4] == 2 && !plain && o->tune[2] == 1)) return false;
+    if (!plain && o->tune[2] > 1) return false;
+    if (!plain && lone && o->tune[2] <= 0 && cells <= kLoneWindowedCells) return false;
+    return j3z::sweeps(shape) && 2 * cells * elem_size(dtype) <= sweep_limit(dtype, shape, o->method);
+}
+
+// Whether the options, or an occupancy that is known, leave one workgroup per CU.
+bool lone_workgroup(const perks_stencil_opts* o, int occupancy)
+{
+    return o->blkpsm == 1 || o->tune[3] == 1 || occupancy == 1;
 }
 
 // Cells a tile of the register-streaming kernels stores, and the ghost planes of a slab.
@@ -197,15 +216,15 @@ int sweep_slabs(int dtype, int nz, long long tiles_xy, int cus, long long waves)
 
 }  // namespace
 
-int j3g_levels(int dtype, int shape, const perks_stencil_opts* o, size_t cells)
+int j3g_levels(int dtype, int shape, const perks_stencil_opts* o, size_t cells, int occupancy)
 {
     const ShapeDesc* sd = shape_by_id(shape);
     if (!sd) return 1;
     if (o->method == PERKS_METHOD_PLAIN) return 1;
     if (use_stream(o, sd->radius)) {
+        if (use_sweep(dtype, shape, o, cells, lone_workgroup(o, occupancy))) return 1;
         const int lm = j3s::stream3_max_levels(sd->radius);
-        if (o->tune[2] <= 0) return use_sweep(dtype, shape, o, 1, cells) ? 1 : lm;
-        return std::min(o->tune[2], lm);
+        return o->tune[2] > 0 ? std::min(o->tune[2], lm) : lm;
     }
     int tx, ty;
     tile_of(dtype, &tx, &ty);
@@ -216,28 +235,25 @@ int j3g_levels(int dtype, int shape, const perks_stencil_opts* o, size_t cells)
     return std::max(1, std::min(L, maxL));
 }
 
-int j3g_plan(int dtype, int nz, int ny, int nx, const perks_stencil_opts* opts, const perks_device_caps* caps,
+int j3g_plan(int dtype, int nz, int ny, int nx, const perks_stencil_opts* o, const perks_device_caps* caps,
              int occupancy, perks_plan_info* out)
 {
-    const ShapeDesc* sd = shape_by_id(opts->shape);
+    const ShapeDesc* sd = shape_by_id(o->shape);
     if (!sd || sd->dims != 3 || !caps || !out) return PERKS_ERR_INVALID_ARG;
-    perks_stencil_opts lim = *opts;
-    if (occupancy == 1) lim.blkpsm = 1;
-    const perks_stencil_opts* o = &lim;
     int tx, ty;
     tile_of(dtype, &tx, &ty);
     const int R = sd->radius;
     const size_t cells = (size_t)nz * ny * nx;
-    const int L = j3g_levels(dtype, o->shape, o, cells);
+    const int L = j3g_levels(dtype, o->shape, o, cells, occupancy);
     if (use_stream(o, R)) {
         const int rows = stream_rows(dtype, R, o);
-        const bool sweep = use_sweep(dtype, o->shape, o, L, cells);
+        const bool sweep = use_sweep(dtype, o->shape, o, cells, lone_workgroup(o, occupancy));
         const TileGeom tg = stream_geom(sweep, R, L, rows);
         const long long tiles_xy = (long long)((nx + tg.vw - 1) / tg.vw) * ((ny + tg.vh - 1) / tg.vh);
         std::memset(out, 0, sizeof(*out));
         out->block = j3s::kWaves * 64;
         out->tile_x = 64;
-        out->tile_y = rows;
+        out->tile_y = sweep ? j3z::kSweepRows + 2 : rows;  // with the ghost rows
         out->reserved[0] = L;
         int nzs = 1;
         long long groups = 0;
@@ -296,9 +312,9 @@ void* j3g_fn(int dtype, const perks_stencil_opts* o, size_t cells, int* block, s
     if (!sd || sd->dims != 3) return nullptr;
     const bool streaming = use_stream(o, sd->radius);
     if (block) *block = streaming ? j3s::kWaves * 64 : j3g::kThreads;
-    if (lds) *lds = streaming ? 0 : lds_for(dtype, sd->radius, j3g_levels(dtype, o->shape, o, cells));
+    if (lds) *lds = streaming ? 0 : lds_for(dtype, sd->radius, j3g_levels(dtype, o->shape, o, cells, 0));
     if (!streaming) return kernel_for(dtype, o->shape, o->boundary);
-    if (use_sweep(dtype, o->shape, o, j3g_levels(dtype, o->shape, o, cells), cells))
+    if (use_sweep(dtype, o->shape, o, cells, lone_workgroup(o, 0)))
         return sweep_kernel_for(dtype, o->shape, o->boundary, o->use_ref_coefs ? sd->divisor != 0.0 : o->divisor != 0.0);
     return stream_kernel_for(dtype, o->shape, o->boundary, stream_rows(dtype, sd->radius, o));
 }
@@ -312,8 +328,9 @@ int j3g_run(int dtype, void* d_a, void* d_b, int nz, int ny, int nx, int steps, 
     const bool streaming = use_stream(o, R);
     const int rows = streaming ? stream_rows(dtype, R, o) : 0;
     const size_t cells = (size_t)nz * ny * nx;
-    const int L = j3g_levels(dtype, o->shape, o, cells);
-    const bool sweep = streaming && use_sweep(dtype, o->shape, o, L, cells);
+    // (the streaming kernels' own occupancy is two or more)
+    const int L = j3g_levels(dtype, o->shape, o, cells, 0);
+    const bool sweep = streaming && use_sweep(dtype, o->shape, o, cells, lone_workgroup(o, 0));
     void* fn = sweep ? sweep_kernel_for(dtype, o->shape, o->boundary, cf.divisor != 0.0)
                      : (streaming ? stream_kernel_for(dtype, o->shape, o->boundary, rows)
                                   : kernel_for(dtype, o->shape, o->boundary));
@@ -411,7 +428,8 @@ int j3g_run(int dtype, void* d_a, void* d_b, int nz, int ny, int nx, int steps, 
         rep->block = threads;
         rep->lds_bytes = (int)lds;
         rep->lds_planes = streaming ? 0 : L * (2 * R + 1);
-        rep->reg_planes = streaming ? (L + 1) * (2 * R + 1) : 0;
+        // (plane by plane: the sums of two planes instead of windows)
+        rep->reg_planes = sweep ? 2 : (streaming ? (L + 1) * (2 * R + 1) : 0);
         rep->occupancy = occ;
         rep->result_in_b = (o->method == PERKS_METHOD_PLAIN ? steps : npass) % 2;
         rep->reserved[0] = L;

@@ -66,11 +66,13 @@ std::vector<Candidate> candidates(int dtype, const perks_stencil_opts* o)
         c.push_back({PERKS_METHOD_PERSISTENT, kResidentVariant, 1});  // resident tiles: one step per barrier
         return c;
     }
-    for (int k : {2, 4, 3}) {  // register streaming (short and tall tiles), LDS planes
+    // register streaming (short and tall tiles; one step per pass of the short one is the
+    // plane-by-plane form where the default takes it), LDS planes
+    for (int k : {2, 4, 3}) {
         c.push_back({PERKS_METHOD_PLAIN, k, 1});
         // the most levels, not the default for a size
         perks_stencil_opts p = with(o, {PERKS_METHOD_PERSISTENT, k, kMaxLevels});
-        const int maxl = j3g_levels(dtype, o->shape, &p, 0);
+        const int maxl = j3g_levels(dtype, o->shape, &p, 0, 0);
         for (int l = 1; l <= maxl; ++l) c.push_back({PERKS_METHOD_PERSISTENT, k, l});
     }
     return c;
