@@ -212,7 +212,8 @@ RowCut cut_rows(int ny, int seg, int edge)
 // update's arithmetic (`ops` per row and lane), by the waves that the fullest
 // SIMD runs (one at a time, or all that are resident in a round) and the rows of
 // an item:
-//   waves * (rows + h)    what the SIMD issues, starting an item h rows' worth;
+//   waves * (rows + h)    what the SIMD issues, starting an item h rows' worth (in a
+//                         batch at least its longest item);
 //   rounds * f / ops      until the first loads of a round have arrived;
 //   e * rows              what the slowest wave takes longer than the others:
 //                         persistent 0.37, under clamp with two or more levels
@@ -229,12 +230,17 @@ RowCut cut_rows(int ny, int seg, int edge)
 //   FP64 5 points 2048^2 per step: 7 rows 356, 16 482, 25 333, 52 362, 97 375
 //   BF16 stochastic 9 points (radius 2) 2048^2 clamp per step: 6 rows 289, 16 299, 36 362
 //   FP16 25 points 2048^2, 2 steps per pass: 12 rows 500, 22 444, 32 536, 72 634
+// In a batch the small grids' items end early and the longest one ends the pass,
+// so rows that only the average counts are not what a height costs: 512 FP32 grids
+// of 64 to 1024 a side, zero, by the longest item 11.4 ms (5 points) and 19.8 (9
+// points), by the average 23.9 and 45.1 (865 workgroups for 1024 places).
 struct PassCost {
     bool plain, tall_dear;
     int cus, occ;
     double h, f, e, lone, ops;
     int trip;
-    double operator()(long long items, double rows) const
+    // rows: of an item on average; most: of the longest one.
+    double operator()(long long items, double rows, double most) const
     {
         const long long simds = 4LL * cus;
         double w = std::ceil((double)((items + kStreamWaves - 1) / kStreamWaves) / cus);
@@ -245,8 +251,8 @@ struct PassCost {
             rounds = (double)((items + simds * occ - 1) / (simds * occ));
             if (rounds > 1) w = rounds * occ;
         }
-        double c = w * (rows + h) + rounds * f / ops + (e + (w == 1 ? lone : 0.0)) * rows;
-        if (tall_dear) c *= 1 + std::max(0.0, 3.7 / ops - 0.07) * std::log(std::max(1.0, rows / trip));
+        double c = std::max(w * (rows + h), most + h) + rounds * f / ops + (e + (w == 1 ? lone : 0.0)) * most;
+        if (tall_dear) c *= 1 + std::max(0.0, 3.7 / ops - 0.07) * std::log(std::max(1.0, most / trip));
         return c;
     }
 };
@@ -290,13 +296,15 @@ int stream_segment(const J2dSpec* specs, int n, int dtype, const ShapeDesc& sd, 
     for (long long k = ghost / trip + 1;; k += 1 + k / (n == 1 ? 16 : 4)) {
         const int seg = (int)std::min<long long>(k * trip - ghost, 0x7fffffffLL);
         long long items = 0;
-        double rows = 0, total = 0;  // rows of the items so far, and of the passes
+        double rows = 0, total = 0;  // rows of the items so far, cost of the passes
+        int longest = 0;             // rows of the longest item so far
         for (size_t i = 0; i < runs.size(); ++i) {
             const long long c = (runs[i].nx + VW - 1LL) / VW * cut_rows(runs[i].ny, seg, edge).count(runs[i].ny);
             items += c;
             rows += (double)c * (std::min(seg, runs[i].ny) + ghost);
+            longest = std::max(longest, std::min(seg, runs[i].ny) + ghost);
             const int next = i + 1 < runs.size() ? runs[i + 1].passes : 0;
-            if (runs[i].passes > next) total += (double)(runs[i].passes - next) * cost(items, rows / (double)items);
+            if (runs[i].passes > next) total += (double)(runs[i].passes - next) * cost(items, rows / (double)items, longest);
         }
         if (total < best_cost * (1 - 1e-9)) {
             best_cost = total;
