@@ -140,6 +140,7 @@ struct CgArgs {
     // lchunk[j] .. lchunk[j+1]-1, chunk c belongs to row j = lcj[c], and
     // lpart[c] receives its value
     const uint8_t* seg_irr;  // CSR: 1 for a segment holding a row of more than kShortRow entries
+    int entries;             // CSR: rowptr[n], for groups_for()
     int balance_nnz;         // CSR with such segments: slots balance entries + rows (else rows)
     int nlong;
     int nchunk;
@@ -1041,10 +1042,12 @@ __global__ void zero_f32(float* __restrict__ d, int n)
 }
 
 // One wave per segment: flags the segments holding a row longer than
-// kShortRow and counts those rows (they are split across the grid).
+// kShortRow and counts those rows (they are split across the grid).  Also
+// passes on the number of entries.
 __global__ void classify_segments(const int32_t* __restrict__ rowptr, int n, int nseg, uint8_t* irr, int* nlong,
-                                  int* nirr)
+                                  int* nirr, int* entries)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *entries = rowptr[n];
     const int lane = threadIdx.x & 63;
     for (int s = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6); s < nseg; s += gridDim.x * (blockDim.x / 64)) {
         int longer = 0, lng = 0;
@@ -1145,6 +1148,7 @@ int ensure(CgScratch& s, size_t n, size_t nval32, int hist_cap)
 struct LongRows {
     int nlong = 0;
     int nchunk = 0;
+    int entries = 0;
     int nirr = 0;  // segments holding rows of more than kShortRow entries
 };
 
@@ -1154,16 +1158,17 @@ struct LongRows {
 int prepare_long_rows(const int32_t* d_rowptr, int n, CgScratch& S, hipStream_t stream, LongRows* out)
 {
     *out = LongRows{};
-    int* d_count = reinterpret_cast<int*>(S.small + 4);  // [0] long rows, [1] irregular segments
+    int* d_count = reinterpret_cast<int*>(S.small + 4);  // [0] long rows, [1] irregular segments, [2] entries
     const int nseg = (n + kSeg - 1) / kSeg;
     PERKS_HIP_TRY(hipMemsetAsync(d_count, 0, 2 * sizeof(int), stream));
     hipLaunchKernelGGL(classify_segments, dim3(std::min(4096, (nseg + 3) / 4)), dim3(256), 0, stream, d_rowptr, n,
-                       nseg, S.seg_irr, d_count, d_count + 1);
+                       nseg, S.seg_irr, d_count, d_count + 1, d_count + 2);
     PERKS_HIP_TRY(hipGetLastError());
-    int counts[2] = {0, 0};
+    int counts[3] = {0, 0, 0};
     PERKS_HIP_TRY(hipMemcpyAsync(counts, d_count, sizeof(counts), hipMemcpyDeviceToHost, stream));
     PERKS_HIP_TRY(hipStreamSynchronize(stream));
     out->nirr = counts[1];
+    out->entries = counts[2];
     const int count = counts[0];
     if (count == 0) return PERKS_OK;
     std::vector<int32_t> rp((size_t)n + 1);
@@ -1204,14 +1209,41 @@ const void* kernel_ptr(int groups)
 {
     switch (groups) {
     case 4: return reinterpret_cast<const void*>(&cg_persistent_kernel<V, FMT, 4>);
-    case 2: return reinterpret_cast<const void*>(&cg_persistent_kernel<V, FMT, 2>);
+    case 2:
+        if constexpr (FMT != FMT_CSR || sizeof(V) < sizeof(double))
+            return reinterpret_cast<const void*>(&cg_persistent_kernel<V, FMT, 2>);
+        [[fallthrough]];
     default: return reinterpret_cast<const void*>(&cg_persistent_kernel<V, FMT, 1>);
     }
 }
 
-// Groups per workgroup: as many as keep every segment in a workgroup of its own
-// with at most kMaxWgPerCu groups per CU.
-int groups_for(int nseg, int cus) { return nseg <= cus ? 4 : (nseg <= 2 * cus ? 2 : 1); }
+// Groups per workgroup.  DIA: as many as keep every segment in a workgroup of its
+// own with at most kMaxWgPerCu groups per CU.  CSR: fewer.  A lane reads its row
+// a chunk at a time, so the lines of a wave's rows have to stay in the caches
+// from one chunk to the next, and with more waves a CU they don't; more groups
+// only gain where rows are one chunk long or the chip is nearly empty.  ms for 60
+// iterations, one, two and four groups (rows of n entries, banded or at random):
+//   FP64  50^3  7 banded  2.36  2.53  2.13     13 banded  3.89  4.69  4.14
+//         80^3  7 banded  2.67  3.36  2.64     19 banded  7.03  9.15  9.33
+//        100^3  7 banded  2.88  3.70  2.92     27 banded 16.9  20.9  19.7
+//        10^6  17 random 32.1  31.5  35.5     39 random  94.5  99.8 111.7
+//       128^3   7 banded  4.43  4.95  5.11      9 random 38.7  44.7  44.1
+//   FP32  50^3  7 banded  2.09  1.66  1.86     27 banded  7.17  6.85  6.71
+//        100^3  7 banded  2.57  2.10  2.53     27 banded 10.7  11.3  11.1
+//         80^3  9 random  7.78  7.98  8.87     13 random 11.3  11.7  11.9
+//       128^3   7 banded  3.55  3.32  4.35     13 random 47.7  48.2  49.6
+template <typename V, int FMT>
+int groups_for(const CgArgs<V>& a, int cus)
+{
+    if constexpr (FMT == FMT_CSR) {
+        const double row = (double)a.entries / a.n;
+        if constexpr (sizeof(V) == sizeof(double)) return row <= kCsrChunk && 2 * a.nseg <= cus ? 4 : 1;
+        if (a.nseg > 2 * cus) return 1;
+        if (a.nseg > cus || row <= 2 * kCsrChunk) return 2;
+        return 8 * a.nseg <= cus ? 4 : 1;
+    }
+    return a.nseg <= cus ? 4 : (a.nseg <= 2 * cus ? 2 : 1);
+}
 
 // The grid and the workgroups' LDS caches.  The grid is CUs x occupancy (at
 // most kMaxWgPerCu per CU, at most one workgroup per segment).  A workgroup
@@ -1241,7 +1273,7 @@ int plan_launch(const CgArgs<V>& a, const perks_cg_opts* o, int* grid, int* grou
     perks_device_caps caps;
     int rc = device_caps_cached(&caps);
     if (rc != PERKS_OK) return rc;
-    const int ng = groups_for(a.nseg, caps.cu_count);
+    const int ng = groups_for<V, FMT>(a, caps.cu_count);
     const void* fn = kernel_ptr<V, FMT>(ng);
     int occ = 0;
     PERKS_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, ng * kLanes, 0));
@@ -1340,6 +1372,7 @@ template <typename V>
 void set_long(CgArgs<V>& a, const CgScratch& S, const LongRows& lr)
 {
     a.seg_irr = S.seg_irr;
+    a.entries = lr.entries;
     a.balance_nnz = lr.nirr > 0 ? 1 : 0;
     a.nlong = lr.nlong;
     a.nchunk = lr.nchunk;
