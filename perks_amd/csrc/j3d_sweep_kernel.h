@@ -17,10 +17,12 @@
 // that traffic, but its 64 x 8 tile then keeps 60 x 4 cells; here a tile keeps
 // all its rows and 62 of 64 columns.
 //
-// ms for 50 steps, persistent, windowed -> here: 27 points 256^3 FP64 4.64 ->
-// 2.70 (311 Gcell/s, 16.5 T FP64 operations/s), FP32 4.50 -> 2.55, bf16 5.56 ->
-// 3.05, 512^3 FP32 27.3 -> 16.3; 17 points 256^3 FP64 3.53 -> 2.16, FP32 3.08 ->
-// 1.61, bf16 3.67 -> 1.99.
+// ms for 50 steps, clamp, windowed -> here.  27 points 256^3 persistent: FP64 4.68 ->
+// 2.77 (303 Gcell/s, 16.0 T FP64 operations/s), FP32 4.54 -> 2.59, bf16 5.69 -> 2.94;
+// per step 4.69 -> 2.51, 3.71 -> 2.28, 4.44 -> 2.48; 512^3 FP32 27.2 -> 17.2, per step
+// 21.5 -> 15.4.  17 points 256^3 persistent: FP64 3.52 -> 2.19, FP32 3.07 -> 1.63, bf16
+// 3.74 -> 1.97; per step 4.36 -> 2.20, 2.75 -> 1.35, 3.14 -> 1.49; 512^3 FP32 17.7 ->
+// 16.2, per step 15.0 both.  100^3 FP64: 27 points 0.76 -> 0.60, 17 points 0.64 -> 0.51.
 //
 // Rows: 4 a tile.  8 read less beyond the tile (512^3 FP32 17-point plain 13.7
 // against 15.5 ms) but make half the waves (64^3 FP64 27-point plain 0.43
