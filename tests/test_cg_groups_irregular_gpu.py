@@ -1,6 +1,6 @@
-"""Irregular CSR systems in each workgroup form of the persistent CG kernel
-(four, two and one groups of 256 lanes to a segment of 4096 rows, by the number
-of segments): hub rows that the grid splits, rows on either side of the split
+"""Irregular CSR systems in the workgroup forms of the persistent CG kernel (four,
+two and one groups of 256 lanes to a segment of 4096 rows, for DIA by the number
+of segments, for CSR by the entries per row as well): hub rows that the grid splits, rows on either side of the split
 length, zero and nonzero starts, FP64, FP32 and refinement, caches on and off.
 A few iterations against the oracle, bit for bit."""
 import numpy as np
