@@ -19,11 +19,11 @@ void release_host_copy();
 // 8 buffers or threads, the same).  The thirds are for a program's first call: with
 // more pieces than three the runtime stands still once for some 6 ms, which the
 // copies of a program that moves little then never pay.  First call of a process
-// (10 steps, FP32 3D) at 8, 16, 24 and 32 MiB: hipMemcpy 6.3, 7.3, 8.5 and 9.2 ms,
-// pieces of 4 MiB 2.9, 10.0, 10.4 and 11.1, thirds 2.3, 4.2, 5.8 and 7.7; the tenth
-// 1.0, 1.8, 2.6, 3.5; 0.83, 1.25, 1.68, 2.0; 0.77, 1.27, 1.70, 2.15.  Beyond, thirds
-// would cost every call for the sake of the first: 48 MiB first call 11.2, 11.5 and
-// 10.9, tenth 5.5, 3.0 and 3.5.
+// (10 steps, FP32 3D) at 8, 16, 24, 30 and 36 MiB: hipMemcpy 6.1, 7.5, 8.4, 9.2 and
+// 10.1 ms, pieces of 4 MiB 2.7, 10.1, 10.4, 10.8 and 11.4, thirds 2.4, 4.2, 5.4, 6.7
+// and 8.2; later ones 0.93, 1.78, 2.84, 3.40 and 4.36; 0.80, 1.25, 1.65, 1.88 and
+// 2.31; 0.68, 1.10, 1.50, 1.84 and 2.46.  Beyond, thirds would cost every call for
+// the sake of the first.
 constexpr int kStagingBuffers = 3;
 constexpr size_t kStagingPiece = (size_t)4 << 20;
 constexpr size_t kStagingThirds = (size_t)36 << 20;

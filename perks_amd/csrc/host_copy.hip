@@ -129,8 +129,12 @@ void map_pages(char* p, size_t bytes)
 }
 
 // One copy in pieces.  Piece c uses buffer c % kBuffers once piece c - kBuffers
-// has left it.  Threads take pieces in order, so of the pieces taken and not done
-// the lowest never waits for one that nobody works on.
+// has left it.  A piece is copied by the host in `slices`, one or a thread's share
+// each: where a copy has three pieces, a thread for each would have the link wait
+// for a whole third at one end.  Host calls of 10 steps FP32 at 16, 24 and 36 MiB,
+// one slice a piece and three: 1.25, 1.76 and 2.72 ms; 1.10, 1.50 and 2.46.
+// Threads take slices in order, so of the slices taken and not done the lowest
+// never waits for one that nobody works on.
 struct Copy {
     Staging* s;
     char* dev;
@@ -139,7 +143,9 @@ struct Copy {
     bool up;  // to the device
     size_t piece_bytes;
     long pieces;
+    long slices;  // of a piece
     std::atomic<long> next{0};
+    std::atomic<long> copied[kBuffers];  // slices of the piece in a buffer that the host has copied
     std::atomic<long> queued[kBuffers];  // pieces queued on the link so far, per buffer
     std::atomic<bool> failed{false};
 
@@ -167,26 +173,36 @@ struct Copy {
         }
         return hipEventSynchronize(s->ev[b]) == hipSuccess;
     }
-    bool piece(long c)
+    // The host's copy of slice q of piece c; the last one of a piece passes the
+    // buffer on to the link.
+    bool slice(long c, long q)
     {
-        char* h = host + (size_t)c * piece_bytes;
+        const size_t share = (piece_bytes / (size_t)slices + 4095) / 4096 * 4096;
+        const size_t from = std::min(size(c), (size_t)q * share);
+        const size_t n = q + 1 < slices ? std::min(share, size(c) - from) : size(c) - from;
+        char* h = host + (size_t)c * piece_bytes + from;
+        char* b = buffer(c) + from;
         if (up) {
             if (c >= kBuffers && !arrived(c - kBuffers)) return false;
-            std::memcpy(buffer(c), h, size(c));
-            return queue(c);
+            std::memcpy(b, h, n);
+        } else {
+            map_pages(h, n);
+            if (!arrived(c)) return false;
+            std::memcpy(h, b, n);
         }
-        map_pages(h, size(c));
-        if (!arrived(c)) return false;
-        std::memcpy(h, buffer(c), size(c));
+        std::atomic<long>& k = copied[c % kBuffers];
+        if (k.fetch_add(1, std::memory_order_acq_rel) + 1 < slices) return true;
+        k.store(0, std::memory_order_relaxed);
+        if (up) return queue(c);
         return c + kBuffers >= pieces || queue(c + kBuffers);
     }
     void work()
     {
         if (hipSetDevice(s->dev) != hipSuccess) failed.store(true);
         for (;;) {
-            const long c = next.fetch_add(1, std::memory_order_relaxed);
-            if (c >= pieces || failed.load(std::memory_order_relaxed)) return;
-            if (!piece(c)) failed.store(true);
+            const long u = next.fetch_add(1, std::memory_order_relaxed);
+            if (u >= pieces * slices || failed.load(std::memory_order_relaxed)) return;
+            if (!slice(u / slices, u % slices)) failed.store(true);
         }
     }
 };
@@ -201,7 +217,9 @@ int staged(Staging* s, char* dev, char* host, size_t bytes, bool up)
     c.up = up;
     c.piece_bytes = staging_piece(s->cap, bytes);
     c.pieces = (long)((bytes + c.piece_bytes - 1) / c.piece_bytes);
+    c.slices = c.pieces <= kBuffers ? kThreads : 1;
     for (auto& q : c.queued) q.store(0);
+    for (auto& k : c.copied) k.store(0);
     if (!up) {
         for (long i = 0; i < std::min<long>(kBuffers, c.pieces); ++i)
             if (!c.queue(i)) c.failed.store(true);
